@@ -271,7 +271,9 @@ static int run_das(const pycbf_rfinfo *info, const float *rf, int64_t nfr, const
     // delay residuals: the direct gather places samples in double
     if (ttx_lo || trx_lo) return launch_das(plan.gk, a, plan.nsplit, part, s);
     if (das_use_plain()) return launch_das_plain(plan.gk, a, s);
-    if (das_reg_applies(plan.gk, nfr, sumflag)) return launch_das_reg(a, s);
+    if (das_wave_applies(plan.gk, a))
+        return launch_das_wave(plan.gk, a, part ? plan.nsplit : 1, part,
+                               plan.bounds ? (int *)cv.take(plan.bounds) : nullptr, s);
     if (plan.bounds) {
         float *bnd = (float *)cv.take(plan.bounds);
         if (!bnd) return fail(PYCBF_EINVAL, "workspace too small");
@@ -281,6 +283,38 @@ static int run_das(const pycbf_rfinfo *info, const float *rf, int64_t nfr, const
     }
     return launch_das(plan.gk, a, plan.nsplit, part, s);
 }
+
+// Tries every significand of [1, 2); rounding to nearest is symmetric in the sign.
+static inline __attribute__((always_inline)) bool recip_scan(float c)
+{
+    const float r = 1.0f / c;
+    for (uint32_t m = 0; m < (1u << 23); m += 1024) {
+        bool ok = true;
+        for (uint32_t k = 0; k < 1024; ++k) {
+            float x;
+            const uint32_t bits = 0x3f800000u | (m + k);
+            memcpy(&x, &bits, 4);
+            const float q = x * r;
+            const float e = __builtin_fmaf(-q, c, x);
+            ok &= (__builtin_fmaf(e, r, q) == x / c);
+        }
+        if (!ok) return false;
+    }
+    return true;
+}
+
+// with the host's fused multiply-adds 2 ms per divisor, through the C library's
+// fma 50 ms
+#if defined(__x86_64__) && !defined(__HIP_DEVICE_COMPILE__)
+__attribute__((target("avx2,fma"))) static bool recip_scan_fma(float c) { return recip_scan(c); }
+static bool recip_scan_host(float c)
+{
+    if (__builtin_cpu_supports("avx2") && __builtin_cpu_supports("fma")) return recip_scan_fma(c);
+    return recip_scan(c);
+}
+#else
+static bool recip_scan_host(float c) { return recip_scan(c); }
+#endif
 
 bool recip_division_exact(float c)
 {
@@ -292,17 +326,7 @@ bool recip_division_exact(float c)
         for (const auto &e : cache)
             if (e.first == c) return e.second;
     }
-    const float r = 1.0f / c;
-    bool ok = true;
-    // every significand of [1, 2); rounding to nearest is symmetric in the sign
-    for (uint32_t m = 0; m < (1u << 23) && ok; ++m) {
-        float x;
-        const uint32_t bits = 0x3f800000u | m;
-        memcpy(&x, &bits, 4);
-        const float q = x * r;
-        const float e = std::fma(-q, c, x);
-        ok = (std::fma(e, r, q) == x / c);
-    }
+    const bool ok = recip_scan_host(c);
     std::lock_guard<std::mutex> lk(mu);
     cache.emplace_back(c, ok);
     return ok;

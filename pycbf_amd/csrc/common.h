@@ -105,10 +105,12 @@ int launch_das(int gk, const DasArgs &a, int nsplit, float *partial, hipStream_t
 // LDS-staged gather (delay tables or in-register synthetic geometry); bounds
 // must hold the tile delay ranges written by launch_tile_bounds.
 int launch_das_lds(int gk, const DasArgs &a, int nsplit, float *partial, hipStream_t s);
-// Single-frame natural-cubic gather with transmit delays in registers: used
-// for one frame summed over tx and rx, or over tx only (das_reg.hip).
-bool das_reg_applies(int gk, int64_t nfr, int sumflag);
-int launch_das_reg(const DasArgs &a, hipStream_t s);
+// Wave-tile gather (das_wave.h): one wave per 64 pixels, samples through L1.
+// It may write up to max_part partial images (nfr, np) into `partial`, and an
+// int of scratch into `fast` (both may be null).
+bool das_wave_applies(int gk, const DasArgs &a);
+int launch_das_wave(int gk, const DasArgs &a, int max_part, float *partial, int *fast,
+                    hipStream_t s);
 // Thread-per-sample gather with one float atomic per contributing sample
 // (pycbf's own GPU launch scheme), the comparator selected by PYCBF_DAS_PLAIN=1.
 bool das_use_plain();

@@ -731,10 +731,8 @@ static void lds_fc(int fc, const DasArgs &a, dim3 grid, hipStream_t s)
 {
     if (fc >= 16)
         lds_geo<GK, SUM, 16>(a.geo, a, grid, s);
-    else if (fc >= 4)
-        lds_geo<GK, SUM, 4>(a.geo, a, grid, s);
     else
-        lds_geo<GK, SUM, 1>(a.geo, a, grid, s);
+        lds_geo<GK, SUM, 4>(a.geo, a, grid, s);
 }
 
 template <int GK>
@@ -755,14 +753,13 @@ static bool das_cubic_dma_enabled()
     return !(e && atoi(e) == 0);
 }
 
-// frames per workgroup for the staged gather: 16, 4 or 1
+// frames per workgroup for the staged gather: 16 or 4 (fewer frames than 4
+// come here only when the wave-tile gather does not take the trace)
 int das_lds_frames_per_pass(int64_t nfr)
 {
     int cap = 16;
     if (const char *e = getenv("PYCBF_DAS_FC")) cap = atoi(e);
-    if (nfr > 8 && cap >= 16) return 16;
-    if (nfr > 1 && cap >= 4) return 4;
-    return 1;
+    return (nfr > 8 && cap >= 16) ? 16 : 4;
 }
 
 int launch_das_lds(int gk, const DasArgs &a0, int nsplit, float *partial, hipStream_t s)

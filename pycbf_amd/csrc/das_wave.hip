@@ -1,0 +1,151 @@
+// Launch of the wave-tile gather (das_wave.h) for nearest and linear, and the
+// rules that pick it and its launch shape for every kind.
+#include <stdlib.h>
+
+#include <algorithm>
+#include <type_traits>
+
+#include "das_wave.h"
+
+namespace pycbf {
+
+int wave_launch_sample(int gk, const DasArgs &a, const WaveArgs &w, int sum, int fc, int mode,
+                       dim3 grid, int nw, size_t lds, hipStream_t s)
+{
+    if (gk == GK_NEAREST) return wave_sum<GK_NEAREST>(sum, fc, mode, a, w, grid, nw, lds, s);
+    return wave_sum<GK_LINEAR>(sum, fc, mode, a, w, grid, nw, lds, s);
+}
+
+bool das_wave_applies(int gk, const DasArgs &a)
+{
+    if (a.nsrc > WAVE_MAX_NSRC || (gk == GK_LINEAR && a.nsrc < 2)) return false;
+    if (a.np > (int64_t)1 << 28) return false;  // 16 threads per pixel within a 32-bit grid
+    // the last sample time must select a knot of the trace
+    if (gk != GK_NEAREST && !((int)((a.tmax - a.t0) / a.dt) <= a.nsrc - 1)) return false;
+    // the cubic over 4 or more frames is staged in LDS (k_das_cubic_dma)
+    return gk != GK_CUBIC || a.nfr < 4;
+}
+
+// Length of the pixel grid's fast axis, read off two delay rows: along a line
+// of pixels the delay to an element outside the line's span changes in one
+// direction, and turns back where the next line starts.  The first turn of
+// either row that divides the pixel count evenly is taken (the longer of the
+// two, 0 when neither does).  Only the grouping of pixels into tiles depends
+// on it, never a result.
+constexpr int FAST_MIN = 32, FAST_MAX = 8192;
+
+__global__ __launch_bounds__(1024) void k_fast_axis(const float *__restrict__ row0,
+                                                    const float *__restrict__ row1, int64_t np,
+                                                    int *__restrict__ fast)
+{
+    __shared__ int turn[2];
+    if (threadIdx.x < 2) turn[threadIdx.x] = FAST_MAX;
+    __syncthreads();
+    const int n = (int)(np < FAST_MAX ? np : FAST_MAX);
+    for (int r = 0; r < 2; ++r) {
+        const float *row = r ? row1 : row0;
+        const float up = row[1] - row[0];
+        int first = FAST_MAX;
+        for (int p = threadIdx.x + 1; p + 1 < n; p += 1024)
+            if (first == FAST_MAX && (row[p + 1] - row[p]) * up < 0.0f) first = p + 1;
+        if (first < FAST_MAX) atomicMin(&turn[r], first);
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        int f = 0;
+        for (int r = 0; r < 2; ++r)
+            if (turn[r] >= FAST_MIN && turn[r] < FAST_MAX && turn[r] > f && np % turn[r] == 0)
+                f = turn[r];
+        *fast = f;
+    }
+}
+
+int launch_fast_axis(const float *ttx, int ntx, const float *trx, int nrx, int64_t np, int *fast,
+                     hipStream_t s)
+{
+    const float *t = nrx >= 2 ? trx : ttx;
+    const int64_t last = (nrx >= 2 ? nrx : ntx) - 1;
+    hipLaunchKernelGGL(k_fast_axis, dim3(1), dim3(1024), 0, s, t, t + last * np, np, fast);
+    return check_launch("fast axis");
+}
+
+int launch_das_wave(int gk, const DasArgs &a0, int max_part, float *partial, int *fast,
+                    hipStream_t s)
+{
+    DasArgs a = a0;
+    WaveArgs w{};
+    // pixels of unknown order over tables: patches of the grid they form
+    // (images of some tiles only; a small one fits the caches in any order)
+    if (a.geo == 0 && !a.perm && fast && a.np >= 4096) {
+        if (int rc = launch_fast_axis(a.ttx, a.ntx, a.trx, a.nrx, a.np, fast, s)) return rc;
+        w.fast = fast;
+    }
+    w.nhalf = (float)a.nsrc - 0.5f;
+    const int sum = a.sumflag == PYCBF_SUM_TX_AND_RX ? WS_BOTH
+                    : a.sumflag == PYCBF_SUM_NONE    ? WS_NONE
+                                                     : WS_SEP;
+    const int fc = a.nfr >= 4 ? 4 : (a.nfr >= 2 ? 2 : 1);
+    int mode = WM_DIV;
+    if (a.rdt == 1.0f / a.dt && recip_division_exact(a.dt))
+        mode = a.t0 == 0.0f ? WM_RECIP0 : WM_RECIP;
+    w.weights = !(a.geo && a.thresh > 0.0f && a.thresh <= 1.0f);
+    const int64_t ntiles = (a.np + 63) / 64;
+    const int64_t passes = (a.nfr + fc - 1) / fc;
+    // Waves per tile: the waves of a tile end together, so many small shares
+    // leave more of them idle at its end, but few tiles need them to fill the
+    // chip.  1024 tiles (31 x 128 x 256 x 256, k-order): 171 us with 8 waves, 152
+    // with 16; 4096 tiles (75 x 128 x 512 x 512, cubic): 845 / 799 / 990 us with
+    // 4 / 8 / 16.
+    int nw = ntiles * passes > 1024 ? 8 : 16;
+    w.group = 1;
+    while (w.group < 32 && ntiles >= 64 * (int64_t)w.group) w.group *= 2;
+    if (sum == WS_BOTH && a.ntx < 8) {
+        // few transmits: the receivers are the inner axis and the waves split them
+        w.inner_tx = 0;
+        w.split_inner = 1;
+    } else {
+        w.inner_tx = a.sumflag != PYCBF_SUM_RX_ONLY;
+    }
+    const int ni = w.inner_tx ? a.ntx : a.nrx, no = w.inner_tx ? a.nrx : a.ntx;
+    if (!w.split_inner)
+        while (nw > 4 && nw / 2 >= no) nw /= 2;
+    const int cap = std::min(WAVE_IB, 160 / (w.weights ? 2 : 1));
+    const int blocks = (ni + cap - 1) / cap;
+    w.ib = blocks == 1 ? ni : ((ni + blocks - 1) / blocks + 15) / 16 * 16;
+    // More workgroups than tiles when the tiles alone leave the chip short of
+    // waves: the outer axis in chunks, whose sums over both axes go through
+    // partial images (as many as the caller's workspace holds).
+    const int64_t waves = ntiles * nw * passes;
+    const int shares = w.split_inner ? no : (no + nw - 1) / nw;
+    int64_t nchunk = std::min<int64_t>((4096 + waves - 1) / waves, shares);
+    if (sum == WS_BOTH) nchunk = std::min<int64_t>(nchunk, partial ? max_part : 1);
+    // Four or more frames read a table too large for the L2s (every XCD would
+    // pull most of it): each XCD takes an eighth of the outer elements instead.
+    // 11 x 127 x 201 x 333, k-order, 12 frames: 600 -> 445 us.
+    if (a.nfr >= 4 && !w.split_inner && sum != WS_NONE && a.np <= (int64_t)1 << 24 &&
+        (sum != WS_BOTH || (partial && max_part >= 8))) {
+        w.slab = 1;
+        nchunk = 8;
+    }
+    float *final_out = a.out;
+    if (sum == WS_BOTH && nchunk > 1) a.out = partial;
+    const size_t lds = std::max((size_t)w.ib * 64 * 4 * (w.weights ? 2 : 1) + (size_t)w.ib * 4 +
+                                    (size_t)nw * 128 * 4,
+                                (size_t)nw * fc * 64 * 4);
+    const dim3 grid((unsigned)(w.slab ? ntiles * 8 : ntiles), (unsigned)(w.slab ? 1 : nchunk),
+                    (unsigned)passes);
+    int rc;
+    {
+        ProfScope prof("das_gather", s);
+        if (gk == GK_CUBIC)
+            rc = wave_launch_cubic(a, w, sum, fc, mode, grid, nw, lds, s);
+        else if (gk == GK_KORDER || gk == GK_AKIMA)
+            rc = wave_launch_hermite(gk, a, w, sum, fc, mode, grid, nw, lds, s);
+        else
+            rc = wave_launch_sample(gk, a, w, sum, fc, mode, grid, nw, lds, s);
+    }
+    if (rc || a.out == final_out) return rc;
+    return launch_reduce_split(partial, (int)nchunk, (int64_t)a.nfr * a.np, final_out, s);
+}
+
+}  // namespace pycbf

@@ -198,11 +198,15 @@ class TabbedBeamformer(Tabbed, GPUBeamformer):
         self._taurx = self._to_dev(self.taurx)
         self._apodtx = self._to_dev(self.apodtx)
         self._apodrx = self._to_dev(self.apodrx)
-        # the gather runs over copies of the tables whose pixel columns are in
-        # a compact processing order (contiguous loads per wave); its image
-        # comes back in that order and is scattered to the pixels' own order
-        self._perm = None
-        self._order = self._to_dev(self._delay_order(), dtype=_torch().int64)
+        # The gather takes the pixels in a compact processing order.  Up to three
+        # frames it reads the tables once per pixel tile and takes that order as
+        # a permutation.  Over more frames it reads them several times (per
+        # channel, or per eighth of the channels): it runs over copies whose
+        # pixel columns are in that order (contiguous loads per wave), and its
+        # image is scattered back to the pixels' own.
+        perm = self._delay_order()
+        self._perm = self._to_dev(perm, dtype=_torch().int32)
+        self._order = self._to_dev(perm, dtype=_torch().int64)
         self._otabs = tuple(t.index_select(1, self._order).contiguous()
                             for t in (self._tautx, self._apodtx, self._taurx, self._apodrx))
         self._obuf = None
@@ -241,16 +245,21 @@ class TabbedBeamformer(Tabbed, GPUBeamformer):
         info = self._rfinfo()
         ws = self._workspace(nframes)
         kind = self.interp["kind"]
-        if self._obuf is None or self._obuf.shape != pout.shape:
-            self._obuf = _torch().empty_like(pout)
-        tt, at, tr, ar = self._otabs
+        ordered = nframes >= 4
+        if ordered:
+            if self._obuf is None or self._obuf.shape != pout.shape:
+                self._obuf = _torch().empty_like(pout)
+            tabs, perm, out = self._otabs, None, self._obuf
+        else:
+            tabs = (self._tautx, self._apodtx, self._taurx, self._apodrx)
+            perm, out = self._perm, pout
         rc = E.lib.pycbf_das_tabbed(
-            ct_byref(info), E.ptr(rf), nframes, E.ptr(tt), E.ptr(at), E.ptr(tr), E.ptr(ar),
-            None, self.nop, E.INTERP[kind], self._interp_param(), E.ptr(self._S_dev()),
-            float(self.thresh), E.SUMTYPE[self.sumtype], E.ptr(self._obuf), E.ptr(ws),
-            ws.numel(), E.stream_of(self._dev))
+            ct_byref(info), E.ptr(rf), nframes, *(E.ptr(t) for t in tabs), E.ptr(perm), self.nop,
+            E.INTERP[kind], self._interp_param(), E.ptr(self._S_dev()), float(self.thresh),
+            E.SUMTYPE[self.sumtype], E.ptr(out), E.ptr(ws), ws.numel(), E.stream_of(self._dev))
         E.check(rc, "pycbf_das_tabbed")
-        pout.index_copy_(pout.dim() - 1, self._order, self._obuf)
+        if ordered:
+            pout.index_copy_(pout.dim() - 1, self._order, out)
 
 
 @dataclass(kw_only=True)

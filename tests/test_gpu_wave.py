@@ -1,0 +1,111 @@
+"""The wave-tile gather (one frame of every kind, several frames of all but the
+cubic) at the sizes where its tiling can go wrong, against the CPU oracle:
+partial and single 64-pixel tiles, few transmits (the waves split the
+receivers), inner axes over one LDS block, two and three frames, passes of
+four with a remainder, a trace start away from zero, weights other than one,
+delays off the trace and NaN.  Bar: 1e-5 of the image peak, as for every image
+(per-sample outputs of nearest and linear bitwise)."""
+import numpy as np
+import pytest
+
+import oracle
+from oracle import numerics
+from pycbf_amd import sim
+from pycbf_amd.gpu import SyntheticBeamformer, TabbedBeamformer
+from tests.helpers import assert_close_to_peak
+
+pytestmark = pytest.mark.gpu
+
+DT = 1.0 / 40e6
+KINDS = [({"kind": "nearest"}, 1), ({"kind": "nearest", "usf": 3}, 3), ({"kind": "linear"}, 1),
+         ({"kind": "cubic"}, 1), ({"kind": "korder_cubic", "k": 8}, 1), ({"kind": "makima"}, 1)]
+# ntx, nrx, np, nfr, t0, unit transmit weights
+SIZES = [(1, 5, 1, None, 0.0, True), (3, 33, 63, 2, 2e-6, False), (7, 16, 64, 3, 0.0, True),
+         (8, 9, 65, None, -1e-6, False), (11, 20, 200, 5, 0.0, True), (170, 6, 130, None, 0.0, True),
+         (90, 3, 70, 4, 1e-6, False), (2, 200, 129, None, 0.0, False)]
+
+
+def _tables(ntx, nrx, npx, nt, t0, unit, rng):
+    span = nt * DT
+    tautx = (t0 + rng.uniform(0.0, 0.5, (ntx, npx)) * span).astype(np.float32)
+    taurx = (rng.uniform(-0.05, 0.6, (nrx, npx)) * span).astype(np.float32)
+    apodtx = np.ones((ntx, npx), np.float32) if unit else rng.uniform(0, 1, (ntx, npx)).astype(np.float32)
+    apodrx = (rng.uniform(0, 1, (nrx, npx)) * (rng.random((nrx, npx)) < 0.7)).astype(np.float32)
+    apodrx[:, ::5] = 0.0  # pixels that no receiver uses
+    taurx[nrx // 2, ::3] = np.nan
+    return tautx, apodtx, taurx, apodrx
+
+
+def _reference(rf, t0, tabs, interp, usf, sumtype, monkeypatch):
+    if interp["kind"] == "makima":
+        # the C oracle has no makima: the thread-per-sample kernel, which places
+        # and evaluates each sample with the same float32 operations
+        monkeypatch.setenv("PYCBF_DAS_PLAIN", "1")
+        out = _beamformer(tabs, t0, rf.shape[-1], interp, sumtype)(rf)
+        monkeypatch.delenv("PYCBF_DAS_PLAIN")
+        return out
+    S = numerics.make_S(8).astype(np.float32) if interp["kind"] == "korder_cubic" else None
+    return np.stack([oracle.das_tabbed(r, t0, DT, *tabs, kind=interp["kind"], usf=usf, sumtype=sumtype, S=S)
+                     for r in rf])
+
+
+def _beamformer(tabs, t0, nt, interp, sumtype):
+    return TabbedBeamformer(tautx=tabs[0], apodtx=tabs[1], taurx=tabs[2], apodrx=tabs[3], t0=t0, dt=DT, nt=nt,
+                            interp=interp, sumtype=sumtype)
+
+
+@pytest.mark.parametrize("interp,usf", KINDS, ids=[k[0]["kind"] + str(k[1]) for k in KINDS])
+@pytest.mark.parametrize("ntx,nrx,npx,nfr,t0,unit", SIZES)
+def test_wave_gather_matches_oracle(ntx, nrx, npx, nfr, t0, unit, interp, usf, monkeypatch):
+    rng = np.random.default_rng(ntx * 1000 + npx)
+    nt = 120
+    tabs = _tables(ntx, nrx, npx, nt, t0, unit, rng)
+    rf = rng.standard_normal((nfr or 1, ntx, nrx, nt)).astype(np.float32)
+    for sumtype in ("tx_and_rx", "tx_only", "rx_only", "none"):
+        print(f"wave {interp} {ntx}x{nrx} {npx} px nfr={nfr} {sumtype}", flush=True)
+        got = _beamformer(tabs, t0, nt, interp, sumtype)(rf if nfr else rf[0])
+        ref = _reference(rf, t0, tabs, interp, usf, sumtype, monkeypatch)
+        ref = ref if nfr else ref[0]
+        if sumtype == "none" and interp["kind"] in ("nearest", "linear") and usf == 1:
+            assert np.array_equal(got, ref.reshape(got.shape))
+        else:
+            assert_close_to_peak(got, ref.reshape(got.shape), 1e-5, sumtype)
+
+
+@pytest.mark.parametrize("thresh", [0.0, 1e-2, 1.5])
+@pytest.mark.parametrize("nfr", [None, 4])
+@pytest.mark.parametrize("kind", ["cubic", "korder_cubic"])
+def test_wave_gather_geometry_equals_its_tables(kind, nfr, thresh):
+    """The point geometry and its own tables select the same samples, at
+    thresholds where zero weights count (0), do not (0.01) and nothing does."""
+    xele = sim.linear_array(24)
+    _, _, pnts = sim.grid(9, 37, (-4e-3, 4e-3), (2e-3, 9e-3))
+    p = sim.pw_synthetic(np.radians(np.linspace(-10, 10, 9)), xele, pnts)
+    rf = np.random.default_rng(4).standard_normal((nfr or 1, 9, 24, 600)).astype(np.float32)
+    rf = rf if nfr else rf[0]
+    kw = dict(t0=0.0, dt=DT, nt=600, interp={"kind": kind}, thresh=thresh)
+    syn = SyntheticBeamformer(**p, **kw)
+    t = syn.tables()
+    tab = TabbedBeamformer(tautx=t[0], apodtx=t[1], taurx=t[2], apodrx=t[3], **kw)
+    a, b = syn(rf), tab(rf)
+    assert_close_to_peak(a, b, 1e-6, f"{kind} thresh={thresh}")
+    assert (thresh > 1.0) == (not np.any(b))
+
+
+@pytest.mark.parametrize("nx,nz,xfast", [(13, 320, False), (64, 64, False), (37, 200, True), (4099, 1, False)])
+def test_wave_gather_over_grids_in_their_own_order(nx, nz, xfast):
+    """Tables handed over in the pixels' own order (das_tabbed): grids of z or
+    x lines, a last band of fewer than eight lines, and pixels that form no
+    grid (a prime count along one line)."""
+    import torch
+    from pycbf_amd.gpu.autograd import das_tabbed
+    xele = sim.linear_array(16)
+    _, _, pnts = sim.grid(nx, nz, (-3e-3, 3e-3), (3e-3, 9e-3))
+    if xfast:
+        pnts = np.ascontiguousarray(pnts.reshape(nx, nz, 2).transpose(1, 0, 2).reshape(-1, 2))
+    tabs = sim.pw_tabs(np.radians([-6.0, 0.0, 4.0]), xele, pnts)
+    rf = np.random.default_rng(9).standard_normal((3, 16, 700)).astype(np.float32)
+    d = lambda a: torch.as_tensor(a, device="cuda")  # noqa: E731
+    for kind in ("cubic", "linear"):
+        got = das_tabbed(d(rf), *(d(t) for t in tabs), 0.0, DT, kind, "tx_and_rx", 1e-2).cpu().numpy()
+        assert_close_to_peak(got, oracle.das_tabbed(rf, 0.0, DT, *tabs, kind=kind), 1e-5, kind)
