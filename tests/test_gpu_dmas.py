@@ -62,3 +62,47 @@ def test_synthetic_dmas_frames():
                                      sumtype="tx_only")
         ref = numerics.dmas(imsep, np.arange(1, 4), "power", True)
         assert_close_to_peak(got[f], ref, 1e-4, f"frame {f}")
+
+
+def _dmas(im, lags, dmastype, sumlags):
+    import torch
+    from pycbf_amd.gpu import _engine as E
+    nfr, nsep, npx = im.shape
+    d = torch.as_tensor(im, device="cuda")
+    L = torch.as_tensor(np.asarray(lags, np.int32), device="cuda")
+    out = torch.empty((nfr, npx) if sumlags else (nfr, len(lags), npx), dtype=torch.float32, device="cuda")
+    E.check(E.lib.pycbf_dmas(E.ptr(d), nfr, nsep, npx, E.ptr(L), len(lags), E.DMASTYPE[dmastype], int(sumlags),
+                             E.ptr(out), E.stream_of(d.device)), "pycbf_dmas")
+    return out.cpu().numpy()
+
+
+@pytest.mark.parametrize("nsep,npx,nfr", [(1, 1, 1), (7, 63, 2), (8, 64, 1), (9, 65, 3), (41, 130, 1), (252, 70, 1),
+                                          (253, 70, 1)])
+def test_dmas_columns_and_lags_at_their_edges(nsep, npx, nfr):
+    """Blocks of eight elements with remainders, columns of 252 elements (the
+    tallest held in LDS) and 253, lags that pair nothing.  Bar: 1e-5 of the
+    peak (float32 sums against FP64)."""
+    im = np.random.default_rng(nsep).standard_normal((nfr, nsep, npx)).astype(np.float32)
+    lags = [1, 0, 3, -2, nsep - 1, nsep, nsep + 5]
+    for dmastype in ("ssr", "power", "pssr"):
+        for sumlags in (True, False):
+            got = _dmas(im, lags, dmastype, sumlags)
+            for f in range(nfr):
+                assert_close_to_peak(got[f], numerics.dmas(im[f], lags, dmastype, sumlags), 1e-5,
+                                     f"{nsep} {dmastype} {sumlags}")
+
+
+def test_dmas_of_infinities_and_nans():
+    """Infinite, NaN and zero elements count as in the column-free kernel, which
+    the same columns padded with zeros to 300 elements take."""
+    rng = np.random.default_rng(1)
+    im = rng.standard_normal((1, 30, 200)).astype(np.float32)
+    for v in (np.inf, -np.inf, np.nan, 0.0):
+        im[0][rng.random((30, 200)) < 0.03] = v
+    tall = np.concatenate([im, np.zeros((1, 270, 200), np.float32)], axis=1)
+    for sumlags in (True, False):
+        got, ref = (_dmas(x, [1, 2, 5], "ssr", sumlags) for x in (im, tall))
+        assert np.array_equal(np.isnan(got), np.isnan(ref)) and np.array_equal(np.isinf(got), np.isinf(ref))
+        fin = np.isfinite(ref)
+        assert np.array_equal(np.sign(got[~fin & ~np.isnan(ref)]), np.sign(ref[~fin & ~np.isnan(ref)]))
+        assert_close_to_peak(got[fin], ref[fin], 1e-5, "finite outputs")
