@@ -6,27 +6,29 @@
 // geometry (pycbf_synthetic_pack), x-major pixel grid, transmit / receive
 // counts and output.  All requests share nt, so their channels are
 // prefiltered by one launch of the natural-spline kernel over the
-// concatenated channel data.  The gather is one persistent kernel: every wave
-// pulls work items (request, TILE x TILE pixel tile, chunk of RC receive
-// elements) from a queue ordered by cost (largest first) through one atomic
-// counter, and exits when the queue is empty.  Within an item a lane owns a
-// pixel; it holds the delays / apodisations of 8 transmits (16 for SLSC
-// requests) in registers while it sweeps the receive chunk (receive geometry
-// evaluated in registers) and gathers the cubic table.  DAS requests add
-// their partial sums into the zeroed image with float atomics; SLSC requests
-// write per-receive images (every (receive element, pixel) is owned by one
-// item), which the per-request SLSC launches then reduce.  Each item stamps
-// its request's completion time (wall clock) for per-request latencies.
+// concatenated channel data.  The gather is one persistent kernel: every
+// workgroup pulls work items (request, TILE x TILE pixel tile, chunk of RC
+// receive elements) from a queue ordered by cost (largest first) through one
+// atomic counter, and exits when the queue is empty.  An item is walked in
+// 8 x 8 pixel patches by the sweep of the wave-tile gather (das_wave.h): the
+// transmits' delays once per patch in LDS, the chunk's receive elements split
+// over the workgroup's waves, elements no pixel of the patch can use dropped.
+// DAS requests add a patch's sum into the zeroed image with one float atomic
+// per pixel; SLSC requests write per-receive images (every (receive element,
+// pixel) is owned by one item), which the per-request SLSC launches then
+// reduce.  64 requests of up to 75 x 256 channels: see the bench; 10 requests of
+// about 31 x 128 x 2048 onto 256 x 256: gather 1.68 -> 0.85 ms (one wave per
+// patch with 8 or 16 transmits in registers before).  Each item stamps its request's completion time (wall clock) for
+// per-request latencies.
 // Every launch of a run is a kernel (no memset), so a run can be captured in
 // a graph.
 #include <math.h>
 
 #include <algorithm>
+#include <type_traits>
 #include <vector>
 
-#include "common.h"
-#include "das_dev.h"
-#include "prof.h"
+#include "das_wave.h"
 
 namespace pycbf {
 
@@ -42,120 +44,110 @@ struct BatchItem {
     int req, tile, r0, pad;
 };
 
-namespace {
+constexpr int BATCH_NW = 4;  // waves per workgroup
 
-// cubic value of channel row `row` at x (0 outside the trace)
-__device__ __forceinline__ float cubic_at(const float *__restrict__ row, float x, const BatchReqDev &R)
+// One item: (tile / 8)^2 patches of 8 x 8 pixels, the receive elements
+// r0 .. r0 + rchunk - 1, all transmits.
+template <int KIND, int MODE>
+__device__ __forceinline__ void batch_item(const BatchReqDev &R, const BatchItem &w, int tile,
+                                           int rchunk, int ib, float *sm, int wave, int lane)
 {
-    int j = 0;
-    if (!knot_index(x, R.t0, R.dt, R.tmax, R.nt, j)) return 0.0f;
-    const float xlead = R.t0 + R.dt * (float)(j + 1);
-    const float xlag = R.t0 + R.dt * (float)j;
-    const float a = (xlead - x) * R.rdt;
-    const float b = (x - xlag) * R.rdt;
-    const float ca = __builtin_fmaf(a * a, a, -a);
-    const float cb = __builtin_fmaf(b * b, b, -b);
-    const Pair2 c = *reinterpret_cast<const Pair2 *>(row + 2 * j);
-    float v = a * c.y0;
-    v = __builtin_fmaf(b, c.y1, v);
-    v = __builtin_fmaf(ca, c.z0, v);
-    return __builtin_fmaf(cb, c.z1, v);
-}
-
-// one work item: TILE x TILE pixels (64 per pass, one per lane), receive
-// elements r0 .. r0+RC-1, all transmits.  Transmits are taken in blocks of
-// BATCH_TB whose delays / apodisations stay in registers while the receive
-// chunk is swept; per-receive images (KIND 1) accumulate in place, since each
-// (receive element, pixel) belongs to this item alone, once per block: they
-// take blocks of 16 (half the read-modify-write passes; the bench batch's
-// best gather 20.46 -> 17.74 ms), summed images 8.
-template <int KIND, int TILE, int RC>
-__device__ __forceinline__ void batch_item(const BatchReqDev &R, int tile, int r0, int lane)
-{
-    constexpr int BATCH_TB = KIND == 1 ? 16 : 8;  // transmits a lane holds in registers
-    const int tiles_z = (R.nz + TILE - 1) / TILE;
-    const int tx0 = (tile / tiles_z) * TILE, tz0 = (tile % tiles_z) * TILE;
-    const int nrc = min(RC, R.nrx - r0);
-    const int64_t np = (int64_t)R.nx * R.nz;
-    const int64_t rowlen = 2 * ((int64_t)R.nt + 1);
-    constexpr int CPP = 64 / TILE;  // tile columns per 64-pixel pass
+    constexpr int SUM = KIND == 0 ? WS_BOTH : WS_SEP;
+    DasArgs A{};
+    A.src = R.coef;
+    A.ch_stride = 2 * ((int64_t)R.nt + 1);
+    A.ntx = R.ntx;
+    A.nrx = R.nrx;
+    A.nfr = 1;
+    A.np = (int64_t)R.nx * R.nz;
+    A.nsrc = R.nt;
+    A.t0 = R.t0;
+    A.dt = R.dt;
+    A.rdt = R.rdt;
+    A.tmax = R.tmax;
+    A.thresh = R.thresh;
+    A.out = R.out;
+    A.geo = 2;
+    A.txpack = R.txpack;
+    A.rxpack = R.rxpack;
+    A.c0 = R.c0;
+    WaveArgs W{};
+    W.ib = ib;
+    W.weights = !(R.thresh > 0.0f && R.thresh <= 1.0f);
+    W.nhalf = (float)R.nt - 0.5f;
+    const int r1 = min(w.r0 + rchunk, R.nrx);
+    WaveShare share;
+    // few transmits: the receive elements are the inner axis and the waves split them
+    const bool few = KIND == 0 && R.ntx < 8;
+    if (few) {
+        share = WaveShare{w.r0, r1, 0, R.ntx, 1, every_nth(wave, BATCH_NW)};
+    } else {
+        W.inner_tx = 1;
+        share = WaveShare{0, R.ntx, w.r0 + wave, r1, BATCH_NW, ~0ull};
+    }
+    const int tiles_z = (R.nz + tile - 1) / tile;
+    const int px0 = (w.tile / tiles_z) * tile, pz0 = (w.tile % tiles_z) * tile;
 #pragma unroll 1
-    for (int pass = 0; pass < TILE / CPP; ++pass) {
-        const int ix = tx0 + pass * CPP + lane / TILE, iz = tz0 + lane % TILE;
-        if (tx0 + pass * CPP >= R.nx) break;  // uniform: the rest of the tile is outside
-        const bool act = ix < R.nx && iz < R.nz;
-        const int64_t p = act ? (int64_t)ix * R.nz + iz : 0;
-        // every lane loads (pixel 0 past the grid), then a full wait: no load
-        // of the position is still counted when the receive loop's gathers are
-        float pv[3] = {R.pvec[2 * p], R.pvec[2 * p + 1], 0.0f};
-        __builtin_amdgcn_s_waitcnt(0);
-        float acc = 0.0f;
+    for (int ox = 0; ox < tile && px0 + ox < R.nx; ox += 8)
 #pragma unroll 1
-        for (int t0 = 0; t0 < R.ntx; t0 += BATCH_TB) {
-            float ttx[BATCH_TB], atx[BATCH_TB];
-#pragma unroll
-            for (int k = 0; k < BATCH_TB; ++k) {
-                ttx[k] = 0.0f;
-                atx[k] = 0.0f;
-                if (t0 + k < R.ntx) {
-                    float pk[PYCBF_TXPACK_FLOATS];
-                    load_pack(R.txpack + (int64_t)(t0 + k) * PYCBF_TXPACK_FLOATS, pk);
-                    geom_tx<2>(pk, R.c0, pv, ttx[k], atx[k]);
+        for (int oz = 0; oz < tile && pz0 + oz < R.nz; oz += 8) {
+            const int ix = px0 + ox + (lane >> 3), iz = pz0 + oz + (lane & 7);
+            const bool act = ix < R.nx && iz < R.nz;
+            const int64_t p = act ? (int64_t)ix * R.nz + iz : 0;
+            const float pv[3] = {R.pvec[2 * p], R.pvec[2 * p + 1], 0.0f};
+            float acc[1] = {0.0f};
+            wave_sweep<GK_CUBIC, SUM, 1, true, MODE>(A, W, sm, share, BATCH_NW, wave, lane, act, p,
+                                                     pv, 0, 1, acc);
+            __syncthreads();  // the patch is done: LDS is free
+            if (KIND == 0) {
+                sm[wave * 64 + lane] = acc[0];
+                __syncthreads();
+                if (wave == 0 && act) {
+                    float s = sm[lane];
+                    for (int v = 1; v < BATCH_NW; ++v) s += sm[v * 64 + lane];
+                    unsafeAtomicAdd(R.out + p, s);
                 }
-            }
-#pragma unroll 1
-            for (int i = 0; i < nrc; ++i) {
-                float trx = 0.0f, arx = 0.0f;
-                float pk[PYCBF_RXPACK_FLOATS];
-                load_pack(R.rxpack + (int64_t)(r0 + i) * PYCBF_RXPACK_FLOATS, pk);
-                geom_rx<2>(pk, R.c0, pv, trx, arx);
-                const float *base = R.coef + ((int64_t)t0 * R.nrx + r0 + i) * rowlen;
-                float part = 0.0f;
-#pragma unroll
-                for (int k = 0; k < BATCH_TB; ++k) {
-                    if (t0 + k >= R.ntx) break;
-                    const float w = atx[k] * arx;
-                    if (act && fabsf(w) >= R.thresh)
-                        part = __builtin_fmaf(
-                            w, cubic_at(base + (int64_t)k * R.nrx * rowlen, ttx[k] + trx, R),
-                            part);
-                }
-                if (KIND == 0) {
-                    acc += part;
-                } else if (act) {
-                    float *o = R.out + (int64_t)(r0 + i) * np + p;
-                    *o = (t0 == 0) ? part : *o + part;
-                }
+                __syncthreads();
             }
         }
-        if (KIND == 0 && act) unsafeAtomicAdd(R.out + p, acc);
-    }
 }
 
-}  // namespace
-
-template <int TILE, int RC>
-__global__ __launch_bounds__(256) void k_batch_das(const BatchReqDev *__restrict__ reqs,
-                                                   const BatchItem *__restrict__ items, int nitems,
-                                                   unsigned *counter,
-                                                   unsigned long long *finish)
+template <int MODE>
+__global__ __launch_bounds__(64 * BATCH_NW) void k_batch_das(const BatchReqDev *__restrict__ reqs,
+                                                             const BatchItem *__restrict__ items,
+                                                             int nitems, unsigned *counter,
+                                                             unsigned long long *finish, int tile,
+                                                             int rchunk, int ib)
 {
+    extern __shared__ float sm[];
+    __shared__ int s_item;
     const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     for (;;) {
-        // every lane executes the atomic, lane 0 adding 1 and the others 0, and
-        // readfirstlane takes lane 0's result into a scalar register: the item
-        // index and the exit test are wave-uniform by construction.  (Pulling
-        // under `if (lane == 0)` let the compiler split the loop on that
-        // loop-invariant lane test, parking lane 0 outside the loop the other
-        // lanes kept running on a stale index.)
-        const unsigned v = atomicAdd(counter, lane == 0 ? 1u : 0u);
-        const int it = (int)__builtin_amdgcn_readfirstlane(v);
-        if (it >= nitems) break;  // every wave leaves once the queue is drained
+        // Wave 0 pulls for the workgroup and passes the item through LDS.  Every
+        // lane of it executes the atomic, lane 0 adding 1 and the others 0, and
+        // the item index and the exit test are uniform by construction.  (Under
+        // `if (threadIdx.x == 0)` the compiler joins the stamp below and this
+        // pull into one branch of lane 0 across the loop's back edge, and parks
+        // that lane outside the loop that the other lanes keep running on a
+        // stale index.)
+        if (wave == 0) {
+            const unsigned v = atomicAdd(counter, lane == 0 ? 1u : 0u);
+            s_item = (int)__builtin_amdgcn_readfirstlane(v);
+        }
+        __syncthreads();
+        const int it = __builtin_amdgcn_readfirstlane(s_item);
+        if (it >= nitems) break;
         const BatchItem w = items[it];
         const BatchReqDev R = reqs[w.req];
-        if (R.kind == 0) batch_item<0, TILE, RC>(R, w.tile, w.r0, lane);
-        else batch_item<1, TILE, RC>(R, w.tile, w.r0, lane);
-        if (lane == 0) atomicMax(finish + w.req, (unsigned long long)wall_clock64());
+        if (R.kind == 0)
+            batch_item<0, MODE>(R, w, tile, rchunk, ib, sm, wave, lane);
+        else
+            batch_item<1, MODE>(R, w, tile, rchunk, ib, sm, wave, lane);
+        // the item ended with a barrier: all of it is done
+        const unsigned long long now = (unsigned long long)wall_clock64();
+        if (wave == 0) atomicMax(finish + w.req, lane == 0 ? now : 0ull);
+        __syncthreads();  // s_item may be written again
     }
 }
 
@@ -187,6 +179,8 @@ struct BatchPlan {
     int nt = 0;
     int tile = 16, rchunk = 32;
     int nitems = 0, max_items = 0;
+    int ib = 1, weights = 0, mode = WM_DIV;  // the gather's LDS block and quotient mode
+    int blocks = 0;                          // resident workgroups of the gather (0: not asked yet)
     float *das_out_base = nullptr;  // DAS outputs are zeroed as one range when contiguous
 };
 
@@ -296,50 +290,35 @@ static int upload(BatchPlan &P, const BatchPtrs &b, hipStream_t s)
     return check(hipStreamSynchronize(s), "batch upload");
 }
 
-// Workgroups of a persistent launch: as many as can be resident at once
-// (every CU times the occupancy the kernel's registers allow), so that the
-// queue is drained by the full complement of waves.
-template <typename K>
-static int persistent_blocks(K kernel)
+template <int MODE>
+static int launch_gather_m(BatchPlan &P, const BatchPtrs &b, hipStream_t s)
 {
-    int dev = 0, cus = 256, per_cu = 0;
-    if (hipGetDevice(&dev) != hipSuccess ||
-        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
-        cus <= 0)
-        cus = 256;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, 256, 0) != hipSuccess ||
-        per_cu < 1)
-        per_cu = 4;
-    return cus * per_cu;
+    const size_t lds = std::max(wave_lds_bytes(P.ib, P.weights, BATCH_NW), (size_t)BATCH_NW * 256);
+    if (!P.blocks) {
+        // as many workgroups as can be resident at once, so that the queue is
+        // drained by the full complement of waves
+        int dev = 0, cus = 256, per_cu = 0;
+        if (hipGetDevice(&dev) != hipSuccess ||
+            hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
+            cus <= 0)
+            cus = 256;
+        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_batch_das<MODE>,
+                                                         64 * BATCH_NW, lds) != hipSuccess ||
+            per_cu < 1)
+            per_cu = 4;
+        P.blocks = cus * per_cu;
+    }
+    hipLaunchKernelGGL(k_batch_das<MODE>, dim3(P.blocks), dim3(64 * BATCH_NW), lds, s, b.reqs,
+                       b.items, P.nitems, b.counter, b.finish, P.tile, P.rchunk, P.ib);
+    return check_launch("batch gather");
 }
 
-template <int TILE, int RC>
-static void launch_gather_t(const BatchPlan &P, const BatchPtrs &b, hipStream_t s)
-{
-    static const int blocks = persistent_blocks(k_batch_das<TILE, RC>);
-    hipLaunchKernelGGL((k_batch_das<TILE, RC>), dim3(blocks), dim3(256), 0, s, b.reqs, b.items,
-                       P.nitems, b.counter, b.finish);
-}
-
-static int launch_gather(const BatchPlan &P, const BatchPtrs &b, hipStream_t s)
+static int launch_gather(BatchPlan &P, const BatchPtrs &b, hipStream_t s)
 {
     ProfScope ps("batch_gather", s);
-    switch (P.tile * 100 + P.rchunk) {
-    case 816: launch_gather_t<8, 16>(P, b, s); break;
-    case 832: launch_gather_t<8, 32>(P, b, s); break;
-    case 864: launch_gather_t<8, 64>(P, b, s); break;
-    case 1616: launch_gather_t<16, 16>(P, b, s); break;
-    case 1632: launch_gather_t<16, 32>(P, b, s); break;
-    case 1664: launch_gather_t<16, 64>(P, b, s); break;
-    case 3216: launch_gather_t<32, 16>(P, b, s); break;
-    case 3232: launch_gather_t<32, 32>(P, b, s); break;
-    case 3264: launch_gather_t<32, 64>(P, b, s); break;
-    case 928: launch_gather_t<8, 128>(P, b, s); break;     // 8 * 100 + 128
-    case 1728: launch_gather_t<16, 128>(P, b, s); break;   // 16 * 100 + 128
-    case 3328: launch_gather_t<32, 128>(P, b, s); break;   // 32 * 100 + 128
-    default: return fail(PYCBF_EINVAL, "unknown gather configuration");
-    }
-    return check_launch("batch gather");
+    if (P.mode == WM_RECIP0) return launch_gather_m<WM_RECIP0>(P, b, s);
+    if (P.mode == WM_RECIP) return launch_gather_m<WM_RECIP>(P, b, s);
+    return launch_gather_m<WM_DIV>(P, b, s);
 }
 
 static int run_batch(BatchPlan &P, const float *rf_all, void *ws, size_t bytes, hipStream_t s,
@@ -421,6 +400,19 @@ int pycbf_batch_create(const pycbf_batch_req *reqs, int nreq, pycbf_batch **out)
         return fail(PYCBF_EINVAL, "DAS outputs must be contiguous, in request order");
     P.nch = chans;
     P.npix_das = das_pix;
+    // One LDS block of inner elements for every request (the transmits, or a
+    // receive chunk of a request with few of them), within 160 rows (weights
+    // take a second array: 80), and one quotient mode that all of them allow.
+    int inner = 1;
+    P.mode = WM_RECIP0;
+    for (const pycbf_batch_req &q : P.reqs) {
+        inner = std::max(inner, q.kind == PYCBF_BATCH_DAS && q.ntx < 8 ? std::min(q.nrx, 128) : q.ntx);
+        if (!(q.thresh > 0.0f && q.thresh <= 1.0f)) P.weights = 1;
+        P.mode = std::min(P.mode, wave_mode_of(q.t0, q.dt, 1.0f / q.dt,
+                                               q.t0 + q.dt * (float)(P.nt - 1), P.nt));
+    }
+    const int cap = P.weights ? 80 : 160, parts = (inner + cap - 1) / cap;
+    P.ib = ((inner + parts - 1) / parts + 15) / 16 * 16;
     for (int t : {8, 16, 32})
         for (int c : {16, 32, 64, 128})
             P.max_items = (int)std::max<int64_t>(P.max_items, items_for(P.reqs, t, c, nullptr));

@@ -69,11 +69,11 @@ __device__ __forceinline__ int64_t band_pixel(int64_t i, int64_t np, int fast)
 // on 31 x 128 x 128 x 1024 per-receive images; 8 costs occupancy.
 constexpr int WAVE_U = 5;
 constexpr int WAVE_IB = 192;  // three 64-bit masks
-// traces this long at most: byte offsets into a row (16 per entry) stay below 2^23
-constexpr int64_t WAVE_MAX_NSRC = (int64_t)1 << 19;
 // A row offset is formed in float: fma(index, bytes, 2^23) holds it in its low
 // bits, in one instruction and with no conversion to integer; the row pointers
-// are lowered by the bits of 2^23.
+// are lowered by the bits of 2^23.  Byte offsets (16 per entry) below 2^23:
+// traces of up to 2^19 entries; longer ones take WM_DIV.
+constexpr int64_t WAVE_FLOAT_NSRC = (int64_t)1 << 19;
 constexpr float WAVE_OFF_BIAS = 8388608.0f;
 constexpr uint32_t WAVE_OFF_BITS = 0x4b000000u;
 
@@ -81,20 +81,34 @@ constexpr uint32_t WAVE_OFF_BITS = 0x4b000000u;
 // (tx, rx) pair
 enum WaveSum { WS_BOTH = 0, WS_SEP = 1, WS_NONE = 2 };
 
-// quotients by dt: the division, products with the reciprocal (dt accepted by
-// recip_division_exact: the same quotients), and those with t0 = 0
+// quotients by dt: the division (with the knot index clamped to the trace, and
+// integer offsets: every trace), products with the reciprocal (dt accepted by
+// recip_division_exact: the same quotients; wave_mode_of says when), and those
+// with t0 = 0
 enum WaveMode { WM_DIV = 0, WM_RECIP = 1, WM_RECIP0 = 2 };
+
+// The mode for a trace of nsrc entries; host only.  The reciprocal modes do not
+// clamp the knot index, so the last sample time itself must select a knot.
+inline int wave_mode_of(float t0, float dt, float rdt, float tmax, int64_t nsrc)
+{
+    if (nsrc > WAVE_FLOAT_NSRC || !((int)((tmax - t0) / dt) <= nsrc - 1)) return WM_DIV;
+    if (rdt != 1.0f / dt || !recip_division_exact(dt)) return WM_DIV;
+    return t0 == 0.0f ? WM_RECIP0 : WM_RECIP;
+}
 
 // a sample's place in its row and what its value needs
 struct WavePos {
-    uint32_t off;         // bytes into the row, plus WAVE_OFF_BITS
+    uint32_t off;         // bytes into the row plus WAVE_OFF_BITS (WM_DIV: the entry)
     float a, b, c, d;     // interpolation weights (or the Hermite position)
     bool in, edge;
 };
 
-__device__ __forceinline__ uint32_t wave_off(float index, float bytes)
+// entry j (jf as a float) of a row with entries of `bytes`
+template <int MODE>
+__device__ __forceinline__ uint32_t wave_off(int j, float jf, float bytes)
 {
-    return __float_as_uint(__builtin_fmaf(index, bytes, WAVE_OFF_BIAS));
+    if (MODE == WM_DIV) return (uint32_t)j;
+    return __float_as_uint(__builtin_fmaf(jf, bytes, WAVE_OFF_BIAS));
 }
 
 // INSIDE: every lane's x is known to lie on the trace
@@ -117,7 +131,8 @@ __device__ __forceinline__ WavePos wave_pos(const DasArgs &A, float nhalf, float
             qc = __builtin_amdgcn_fmed3f(q, 0.0f, nhalf - 0.5f);
         }
         const float jf = truncf(qc);
-        P.off = wave_off((qc - jf >= 0.5f) ? jf + 1.0f : jf, 4.0f);
+        const float it = (qc - jf >= 0.5f) ? jf + 1.0f : jf;
+        P.off = wave_off<MODE>((int)it, it, 4.0f);
         return P;
     }
     float xc = x;
@@ -126,15 +141,15 @@ __device__ __forceinline__ WavePos wave_pos(const DasArgs &A, float nhalf, float
         P.in = xc == x;
     }
     const float q = over_dt(MODE == WM_RECIP0 ? xc : xc - t0);
-    // the launch checks that tmax itself selects a knot below nsrc
-    const float jf = truncf(q);
+    const int j = MODE == WM_DIV ? min((int)q, A.nsrc - 1) : 0;
+    const float jf = MODE == WM_DIV ? (float)j : truncf(q);
     if (GK == GK_KORDER || GK == GK_AKIMA) {
         if (MODE == WM_RECIP0)
             P.a = (xc - A.dt * jf) * A.rdt;
         else
             P.a = (GK == GK_KORDER) ? ((xc - t0) - A.dt * jf) * A.rdt
                                     : (xc - (t0 + A.dt * jf)) * A.rdt;
-        P.off = wave_off(jf, 16.0f);
+        P.off = wave_off<MODE>(j, jf, 16.0f);
         return P;
     }
     const float lead = A.dt * (jf + 1.0f), lag = A.dt * jf;
@@ -145,15 +160,15 @@ __device__ __forceinline__ WavePos wave_pos(const DasArgs &A, float nhalf, float
         P.b = EXACT ? over_dt(xc - xlag) : (xc - xlag) * A.rdt;
         // the pair (nsrc - 2, nsrc - 1) serves the last knot, whose successor is 0
         const float last = nhalf - 1.5f;
-        P.edge = jf > last;
-        P.off = wave_off(fminf(jf, last), 4.0f);
+        P.edge = MODE == WM_DIV ? j > A.nsrc - 2 : jf > last;
+        P.off = wave_off<MODE>(min(j, A.nsrc - 2), fminf(jf, last), 4.0f);
         return P;
     }
     P.a = (xlead - xc) * A.rdt;
     P.b = (xc - xlag) * A.rdt;
     P.c = __builtin_fmaf(P.a * P.a, P.a, -P.a);
     P.d = __builtin_fmaf(P.b * P.b, P.b, -P.b);
-    P.off = wave_off(jf, 8.0f);
+    P.off = wave_off<MODE>(j, jf, 8.0f);
     return P;
 }
 
@@ -162,33 +177,39 @@ typedef __attribute__((address_space(3))) float lds_float;
 struct WaveRaw {
     float v[4];
 };
-struct __attribute__((aligned(4))) WavePair {
-    float y0, y1;
-};
+// a row's entries as read: pairs at 4-byte, (y, h*y2) pairs at 8-byte alignment
+typedef float wave_f2 __attribute__((ext_vector_type(2), aligned(4)));
+typedef float wave_f4a8 __attribute__((ext_vector_type(4), aligned(8)));
+typedef float wave_f4 __attribute__((ext_vector_type(4), aligned(16)));
 
-template <int GK>
-__device__ __forceinline__ WaveRaw wave_load(const char *row, uint32_t off)
+template <int GK, int MODE>
+__device__ __forceinline__ WaveRaw wave_load(const char *row, uint32_t o)
 {
+    constexpr int BYTES = GK == GK_CUBIC ? 8 : (GK == GK_KORDER || GK == GK_AKIMA ? 16 : 4);
+    // rows are global memory, also where the compiler cannot see it
+#define WAVE_AT(T) (*(const __attribute__((address_space(1))) T *)((uintptr_t)row + off))
+    const size_t off = MODE == WM_DIV ? (size_t)o * BYTES + WAVE_OFF_BITS : (size_t)o;
     WaveRaw r;
     if (GK == GK_NEAREST) {
-        r.v[0] = *reinterpret_cast<const float *>(row + off);
+        r.v[0] = WAVE_AT(float);
     } else if (GK == GK_LINEAR) {
-        const WavePair p = *reinterpret_cast<const WavePair *>(row + off);
-        r.v[0] = p.y0;
-        r.v[1] = p.y1;
+        const wave_f2 p = WAVE_AT(wave_f2);
+        r.v[0] = p.x;
+        r.v[1] = p.y;
     } else if (GK == GK_CUBIC) {
-        const Pair2 p = *reinterpret_cast<const Pair2 *>(row + off);
-        r.v[0] = p.y0;
-        r.v[1] = p.z0;
-        r.v[2] = p.y1;
-        r.v[3] = p.z1;
+        const wave_f4a8 p = WAVE_AT(wave_f4a8);  // y_j, z_j, y_j+1, z_j+1
+        r.v[0] = p.x;
+        r.v[1] = p.y;
+        r.v[2] = p.z;
+        r.v[3] = p.w;
     } else {
-        const float4 p = *reinterpret_cast<const float4 *>(row + off);
+        const wave_f4 p = WAVE_AT(wave_f4);
         r.v[0] = p.x;
         r.v[1] = p.y;
         r.v[2] = p.z;
         r.v[3] = p.w;
     }
+#undef WAVE_AT
     return r;
 }
 
@@ -228,10 +249,37 @@ __device__ __forceinline__ float wave_value(const WavePos &P, const WaveRaw &r)
                           r.v[0]);
 }
 
-template <int GK, int SUM, int FC, bool GEOM, int MODE>
-__global__ __launch_bounds__(1024) void k_das_wave(DasArgs A, WaveArgs W)
+// This wave's share of a tile's channels: inner elements ibeg .. iend - 1 (held
+// in LDS by the whole workgroup, of which it takes those in `pat`), outer ones
+// obeg, obeg + ostep, ... below oend.
+struct WaveShare {
+    int ibeg, iend, obeg, oend, ostep;
+    uint64_t pat;
+};
+
+__device__ __forceinline__ uint64_t every_nth(int wave, int nw)
 {
-    extern __shared__ float sm[];
+    uint64_t pat = 1ull << wave;
+    for (int s = nw; s < 64; s <<= 1) pat |= pat << s;
+    return pat;
+}
+
+// LDS of one workgroup: delays (and weights) of ib inner elements, the waves'
+// delay ranges, the elements' flags
+__host__ __device__ inline size_t wave_lds_bytes(int ib, int weights, int nw)
+{
+    return (size_t)ib * 64 * 4 * (weights ? 2 : 1) + (size_t)nw * 128 * 4 + (size_t)ib * 4;
+}
+
+// Walks the workgroup's tile (this lane's pixel p at pv): sums of both axes go
+// to acc, the other classes to A.out.  All waves of the workgroup call it
+// together, and LDS is free when they do.
+template <int GK, int SUM, int FC, bool GEOM, int MODE>
+__device__ __forceinline__ void wave_sweep(const DasArgs &A, const WaveArgs &W, float *sm,
+                                           const WaveShare &share, int nw, int wave, int lane,
+                                           bool act, int64_t p, const float (&pv)[3], int f0,
+                                           int nf, float (&acc)[FC])
+{
     constexpr int U = FC == 1 ? WAVE_U : (FC == 2 ? 2 : 1);  // channels in flight together
     constexpr bool EXACT = SUM == WS_NONE;
     // Single-frame images of one element feed the coherence kernels, whose
@@ -239,6 +287,198 @@ __global__ __launch_bounds__(1024) void k_das_wave(DasArgs A, WaveArgs W)
     // the order of these sums is part of the result (whole values, added in
     // blocks of 16 inner elements, the blocks then added in order).
     constexpr bool B16 = SUM == WS_SEP && GK == GK_CUBIC && FC == 1;
+    constexpr int GEO = GEOM ? 3 : 0;
+    const bool inner_tx = W.inner_tx != 0;
+    const int no = inner_tx ? A.nrx : A.ntx;
+    const bool drop = A.thresh > 0.0f;  // a zero (or NaN) weight then never contributes
+    float *s_tau = sm;
+    float *s_wgt = sm + W.ib * 64;
+    // this lane's column of s_tau as an LDS address the compiler holds in one
+    // register (it would add the array's base again for every channel)
+    uint32_t l_tau = (uint32_t)(uintptr_t)(lds_float *)(s_tau + lane);
+    asm("" : "+v"(l_tau));
+    auto tau_of = [&](int k) { return *(lds_float *)(uintptr_t)(l_tau + ((uint32_t)k << 8)); };
+    float *s_rng = sm + W.ib * 64 * (W.weights ? 2 : 1);  // (nw, 64) delay ranges (lo, hi)
+    int *s_flag = reinterpret_cast<int *>(s_rng + nw * 128);
+    const int64_t fbytes = (int64_t)A.ntx * A.nrx * A.ch_stride * 4;
+    const int64_t ibytes = (inner_tx ? (int64_t)A.nrx : 1) * A.ch_stride * 4;
+    const int64_t obytes = (inner_tx ? 1 : (int64_t)A.nrx) * A.ch_stride * 4;
+
+    for (int i0 = share.ibeg; i0 < share.iend; i0 += W.ib) {
+        const int n = min(W.ib, share.iend - i0);
+        if (i0 != share.ibeg) __syncthreads();
+        float lo = INFINITY, hi = -INFINITY;  // this lane's delays over the kept elements
+        for (int k = wave; k < n; k += nw) {
+            float tau, ap;
+            elem_eval<GEO>(A, inner_tx, i0 + k, p, pv, tau, ap);
+            if (!act || (drop && !(ap != 0.0f && ap == ap))) tau = NAN;
+            s_tau[k * 64 + lane] = tau;
+            if (W.weights) s_wgt[k * 64 + lane] = ap;
+            const int any = __any(tau == tau) ? 1 : 0;
+            const int ones = __all(!(tau == tau) || ap == 1.0f) ? 2 : 0;
+            if (lane == 0) s_flag[k] = any | ones;
+            if (any) {
+                lo = (tau == tau) ? fminf(lo, tau) : -INFINITY;
+                hi = (tau == tau) ? fmaxf(hi, tau) : INFINITY;
+            }
+        }
+        s_rng[wave * 128 + lane] = lo;
+        s_rng[wave * 128 + 64 + lane] = hi;
+        __syncthreads();
+        for (int v = 0; v < nw; ++v) {
+            lo = fminf(lo, s_rng[v * 128 + lane]);
+            hi = fmaxf(hi, s_rng[v * 128 + 64 + lane]);
+        }
+        uint64_t mask[WAVE_IB / 64];
+        bool unit = true;
+#pragma unroll
+        for (int w = 0; w < WAVE_IB / 64; ++w) {
+            const int fl = (w * 64 + lane < n) ? s_flag[w * 64 + lane] : 2;
+            const uint64_t m = __ballot((SUM == WS_NONE) ? (w * 64 + lane < n) : (fl & 1) != 0) & share.pat;
+            mask[w] = ((uint64_t)__builtin_amdgcn_readfirstlane((uint32_t)(m >> 32)) << 32) |
+                      (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)m);
+            unit = unit && __all((fl & 2) != 0);
+        }
+        // all inner weights 1 (or their lanes dropped): samples are summed
+        // unweighted and the outer weight is applied to the sum
+        if (!W.weights) unit = true;
+
+        for (int o = share.obeg; o < share.oend; o += share.ostep) {
+            float to, wo;
+            elem_eval<GEO>(A, !inner_tx, o, p, pv, to, wo);
+            if (!act || (drop && !(wo != 0.0f && wo == wo))) to = NAN;
+            if (unit && !(fabsf(wo) >= A.thresh)) to = NAN;
+            float part[FC];
+#pragma unroll
+            for (int f = 0; f < FC; ++f) part[f] = 0.0f;
+            const char *row0 = reinterpret_cast<const char *>(A.src) + (int64_t)f0 * fbytes +
+                               (int64_t)i0 * ibytes + (int64_t)o * obytes;
+            float total = 0.0f;  // B16: the sum of the blocks before k's
+            int block = 0;
+            // nu channels: positions, then every load, then the values
+            auto group = [&](const int *k, auto nuc, auto kindc) {
+                constexpr int NU = decltype(nuc)::value;
+                constexpr bool UNIT = decltype(kindc)::value >= 1;
+                constexpr bool INSIDE = decltype(kindc)::value == 2;
+                WavePos P[NU];
+                WaveRaw R[NU][FC];
+                float wgt[NU];
+#pragma unroll
+                for (int u = 0; u < NU; ++u) {
+                    P[u] = wave_pos<GK, MODE, EXACT, INSIDE>(A, W.nhalf, tau_of(k[u]) + to);
+                    wgt[u] = 1.0f;
+                    if (!UNIT) {
+                        wgt[u] = s_wgt[k[u] * 64 + lane] * wo;  // apodtx * apodrx
+                        P[u].in = P[u].in && fabsf(wgt[u]) >= A.thresh;
+                    }
+                }
+#pragma unroll
+                for (int u = 0; u < NU; ++u) {
+                    const char *row = row0 + (int64_t)k[u] * ibytes - WAVE_OFF_BITS;
+#pragma unroll
+                    for (int f = 0; f < FC; ++f)
+                        R[u][f] = wave_load<GK, MODE>(row + (int64_t)min(f, nf - 1) * fbytes, P[u].off);
+                }
+#pragma unroll
+                for (int u = 0; u < NU; ++u) {
+                    if (B16 && (k[u] >> 4) != block) {  // wave-uniform
+                        block = k[u] >> 4;
+                        total += part[0];
+                        part[0] = 0.0f;
+                    }
+#pragma unroll
+                    for (int f = 0; f < FC; ++f) {
+                        if (SUM == WS_NONE) {
+                            const float v = wave_value<GK, EXACT>(P[u], R[u][f]);
+                            const int e = i0 + k[u];
+                            const int64_t ch = inner_tx ? (int64_t)e * A.nrx + o
+                                                        : (int64_t)o * A.nrx + e;
+                            const float w = UNIT ? (GEOM ? 1.0f : wo) : wgt[u];
+                            if (act && f < nf)
+                                A.out[((int64_t)(f0 + f) * A.ntx * A.nrx + ch) * A.np + p] =
+                                    P[u].in ? 0.0f + w * v : 0.0f;
+                        } else if (INSIDE) {
+                            part[f] = wave_add<GK, !B16>(P[u], R[u][f], part[f]);
+                        } else if (UNIT) {
+                            const float s = wave_add<GK, !B16>(P[u], R[u][f], part[f]);
+                            part[f] = P[u].in ? s : part[f];
+                        } else {
+                            const float v = wave_value<GK, EXACT>(P[u], R[u][f]);
+                            const float s = __builtin_fmaf(wgt[u], v, part[f]);
+                            part[f] = P[u].in ? s : part[f];
+                        }
+                    }
+                }
+            };
+            auto sweep = [&](auto kindc) {
+#pragma unroll 1
+                for (int w = 0; w < WAVE_IB / 64; ++w) {
+                    uint64_t m = w == 0 ? mask[0] : (w == 1 ? mask[1] : mask[2]);
+                    int left = __popcll(m);
+                    int k[U];
+                    for (; left >= U; left -= U) {
+#pragma unroll
+                        for (int u = 0; u < U; ++u) {
+                            k[u] = w * 64 + __builtin_ctzll(m);
+                            m &= m - 1;
+                        }
+                        group(k, std::integral_constant<int, U>(), kindc);
+                    }
+                    for (; U > 2 && left >= 2; left -= 2) {
+#pragma unroll
+                        for (int u = 0; u < 2; ++u) {
+                            k[u] = w * 64 + __builtin_ctzll(m);
+                            m &= m - 1;
+                        }
+                        group(k, std::integral_constant<int, (U > 2 ? 2 : 1)>(), kindc);
+                    }
+                    for (; left > 0; --left) {
+                        k[0] = w * 64 + __builtin_ctzll(m);
+                        m &= m - 1;
+                        group(k, std::integral_constant<int, 1>(), kindc);
+                    }
+                }
+                if (B16) part[0] = total + part[0];
+            };
+            if (SUM == WS_NONE || __any(to == to)) {
+                // every sample of the wave on the trace: no clamps, no selects
+                const bool inside = SUM != WS_NONE && unit &&
+                                    __all(lo + to >= A.t0 && hi + to <= A.tmax);
+                if (inside)
+                    sweep(std::integral_constant<int, SUM == WS_NONE ? 1 : 2>());
+                else if (unit)
+                    sweep(std::integral_constant<int, 1>());
+                else
+                    sweep(std::integral_constant<int, 0>());
+            }
+            if (SUM == WS_NONE) continue;
+            if (!GEOM && unit) {
+#pragma unroll
+                for (int f = 0; f < FC; ++f) part[f] *= (to == to) ? wo : 0.0f;
+            }
+            if (SUM == WS_BOTH) {
+#pragma unroll
+                for (int f = 0; f < FC; ++f) acc[f] += part[f];
+            } else if (act) {
+#pragma unroll
+                for (int f = 0; f < FC; ++f)
+                    if (f < nf) {
+                        float *q = A.out + ((int64_t)(f0 + f) * no + o) * A.np + p;
+                        *q = (i0 == share.ibeg) ? part[f] : *q + part[f];
+                    }
+            }
+        }
+    }
+}
+
+// eight waves per SIMD (64 VGPRs, some scalars kept in vector lanes outside the
+// inner loop) measured 793 -> 768 us against the compiler's own seven on
+// 75 x 128 x 512 x 512, cubic
+template <int GK, int SUM, int FC, bool GEOM, int MODE>
+__global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(8))) void
+k_das_wave(DasArgs A, WaveArgs W)
+{
+    extern __shared__ float sm[];
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int nw = blockDim.x >> 6;
@@ -283,191 +523,15 @@ __global__ __launch_bounds__(1024) void k_das_wave(DasArgs A, WaveArgs W)
             else pv[2] = v;
         }
     }
-    constexpr int GEO = GEOM ? 3 : 0;
-    const bool inner_tx = W.inner_tx != 0;
-    const int ni = inner_tx ? A.ntx : A.nrx, no = inner_tx ? A.nrx : A.ntx;
-    const bool drop = A.thresh > 0.0f;  // a zero (or NaN) weight then never contributes
-    float *s_tau = sm;
-    float *s_wgt = sm + W.ib * 64;
-    // this lane's column of s_tau as an LDS address the compiler holds in one
-    // register (it would add the array's base again for every channel)
-    uint32_t l_tau = (uint32_t)(uintptr_t)(lds_float *)(s_tau + lane);
-    asm("" : "+v"(l_tau));
-    auto tau_of = [&](int k) { return *(lds_float *)(uintptr_t)(l_tau + ((uint32_t)k << 8)); };
-    float *s_rng = sm + W.ib * 64 * (W.weights ? 2 : 1);  // (nw, 64) delay ranges (lo, hi)
-    int *s_flag = reinterpret_cast<int *>(s_rng + nw * 128);
-    const int o0 = W.split_inner ? chunk : chunk + nchunk * wave;
-    const int os = W.split_inner ? nchunk : nchunk * nw;
-    // this wave's share of a block's inner elements: every nw-th one
-    uint64_t pat = ~0ull;
-    if (W.split_inner) {
-        pat = 1ull << wave;
-        for (int s = nw; s < 64; s <<= 1) pat |= pat << s;
-    }
-    const int64_t fbytes = (int64_t)A.ntx * A.nrx * A.ch_stride * 4;
-    const int64_t ibytes = (inner_tx ? (int64_t)A.nrx : 1) * A.ch_stride * 4;
-    const int64_t obytes = (inner_tx ? 1 : (int64_t)A.nrx) * A.ch_stride * 4;
+    const bool itx = W.inner_tx != 0;
+    WaveShare share{0, itx ? A.ntx : A.nrx, W.split_inner ? chunk : chunk + nchunk * wave,
+                    itx ? A.nrx : A.ntx, W.split_inner ? nchunk : nchunk * nw, ~0ull};
+    if (W.split_inner) share.pat = every_nth(wave, nw);
 
     float acc[FC];
 #pragma unroll
     for (int f = 0; f < FC; ++f) acc[f] = 0.0f;
-
-    for (int i0 = 0; i0 < ni; i0 += W.ib) {
-        const int n = min(W.ib, ni - i0);
-        if (i0) __syncthreads();
-        float lo = INFINITY, hi = -INFINITY;  // this lane's delays over the kept elements
-        for (int k = wave; k < n; k += nw) {
-            float tau, ap;
-            elem_eval<GEO>(A, inner_tx, i0 + k, p, pv, tau, ap);
-            if (!act || (drop && !(ap != 0.0f && ap == ap))) tau = NAN;
-            s_tau[k * 64 + lane] = tau;
-            if (W.weights) s_wgt[k * 64 + lane] = ap;
-            const int any = __any(tau == tau) ? 1 : 0;
-            const int ones = __all(!(tau == tau) || ap == 1.0f) ? 2 : 0;
-            if (lane == 0) s_flag[k] = any | ones;
-            if (any) {
-                lo = (tau == tau) ? fminf(lo, tau) : -INFINITY;
-                hi = (tau == tau) ? fmaxf(hi, tau) : INFINITY;
-            }
-        }
-        s_rng[wave * 128 + lane] = lo;
-        s_rng[wave * 128 + 64 + lane] = hi;
-        __syncthreads();
-        for (int v = 0; v < nw; ++v) {
-            lo = fminf(lo, s_rng[v * 128 + lane]);
-            hi = fmaxf(hi, s_rng[v * 128 + 64 + lane]);
-        }
-        uint64_t mask[WAVE_IB / 64];
-        bool unit = true;
-#pragma unroll
-        for (int w = 0; w < WAVE_IB / 64; ++w) {
-            const int fl = (w * 64 + lane < n) ? s_flag[w * 64 + lane] : 2;
-            const uint64_t m = __ballot((SUM == WS_NONE) ? (w * 64 + lane < n) : (fl & 1) != 0) & pat;
-            mask[w] = ((uint64_t)__builtin_amdgcn_readfirstlane((uint32_t)(m >> 32)) << 32) |
-                      (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)m);
-            unit = unit && __all((fl & 2) != 0);
-        }
-        // all inner weights 1 (or their lanes dropped): samples are summed
-        // unweighted and the outer weight is applied to the sum
-        if (!W.weights) unit = true;
-
-        for (int o = o0; o < no; o += os) {
-            float to, wo;
-            elem_eval<GEO>(A, !inner_tx, o, p, pv, to, wo);
-            if (!act || (drop && !(wo != 0.0f && wo == wo))) to = NAN;
-            if (unit && !(fabsf(wo) >= A.thresh)) to = NAN;
-            float part[FC];
-#pragma unroll
-            for (int f = 0; f < FC; ++f) part[f] = 0.0f;
-            const char *row0 = reinterpret_cast<const char *>(A.src) + (int64_t)f0 * fbytes +
-                               (int64_t)i0 * ibytes + (int64_t)o * obytes;
-            // nu channels: positions, then every load, then the values
-            auto group = [&](const int *k, auto nuc, auto kindc) {
-                constexpr int NU = decltype(nuc)::value;
-                constexpr bool UNIT = decltype(kindc)::value >= 1;
-                constexpr bool INSIDE = decltype(kindc)::value == 2;
-                WavePos P[NU];
-                WaveRaw R[NU][FC];
-                float wgt[NU];
-#pragma unroll
-                for (int u = 0; u < NU; ++u) {
-                    P[u] = wave_pos<GK, MODE, EXACT, INSIDE>(A, W.nhalf, tau_of(k[u]) + to);
-                    wgt[u] = 1.0f;
-                    if (!UNIT) {
-                        wgt[u] = s_wgt[k[u] * 64 + lane] * wo;  // apodtx * apodrx
-                        P[u].in = P[u].in && fabsf(wgt[u]) >= A.thresh;
-                    }
-                }
-#pragma unroll
-                for (int u = 0; u < NU; ++u) {
-                    const char *row = row0 + (int64_t)k[u] * ibytes - WAVE_OFF_BITS;
-#pragma unroll
-                    for (int f = 0; f < FC; ++f)
-                        R[u][f] = wave_load<GK>(row + (int64_t)min(f, nf - 1) * fbytes, P[u].off);
-                }
-#pragma unroll
-                for (int u = 0; u < NU; ++u)
-#pragma unroll
-                    for (int f = 0; f < FC; ++f) {
-                        if (SUM == WS_NONE) {
-                            const float v = wave_value<GK, EXACT>(P[u], R[u][f]);
-                            const int e = i0 + k[u];
-                            const int64_t ch = inner_tx ? (int64_t)e * A.nrx + o
-                                                        : (int64_t)o * A.nrx + e;
-                            const float w = UNIT ? (GEOM ? 1.0f : wo) : wgt[u];
-                            if (act && f < nf)
-                                A.out[((int64_t)(f0 + f) * A.ntx * A.nrx + ch) * A.np + p] =
-                                    P[u].in ? 0.0f + w * v : 0.0f;
-                        } else if (INSIDE) {
-                            part[f] = wave_add<GK, !B16>(P[u], R[u][f], part[f]);
-                        } else if (UNIT) {
-                            const float s = wave_add<GK, !B16>(P[u], R[u][f], part[f]);
-                            part[f] = P[u].in ? s : part[f];
-                        } else {
-                            const float v = wave_value<GK, EXACT>(P[u], R[u][f]);
-                            const float s = __builtin_fmaf(wgt[u], v, part[f]);
-                            part[f] = P[u].in ? s : part[f];
-                        }
-                    }
-            };
-            auto sweep = [&](auto kindc) {
-                float total = 0.0f;  // B16: the blocks' sum
-#pragma unroll 1
-                for (int g = 0; g < WAVE_IB / 64 * (B16 ? 4 : 1); ++g) {
-                    const int w = B16 ? g >> 2 : g, base = B16 ? g * 16 : g * 64;
-                    uint64_t m = w == 0 ? mask[0] : (w == 1 ? mask[1] : mask[2]);
-                    if (B16) m = (m >> (16 * (g & 3))) & 0xffffu;
-                    int left = __popcll(m);
-                    int k[U];
-                    for (; left >= U; left -= U) {
-#pragma unroll
-                        for (int u = 0; u < U; ++u) {
-                            k[u] = base + __builtin_ctzll(m);
-                            m &= m - 1;
-                        }
-                        group(k, std::integral_constant<int, U>(), kindc);
-                    }
-                    for (; left > 0; --left) {
-                        k[0] = base + __builtin_ctzll(m);
-                        m &= m - 1;
-                        group(k, std::integral_constant<int, 1>(), kindc);
-                    }
-                    if (B16) {
-                        total += part[0];
-                        part[0] = 0.0f;
-                    }
-                }
-                if (B16) part[0] = total;
-            };
-            if (SUM == WS_NONE || __any(to == to)) {
-                // every sample of the wave on the trace: no clamps, no selects
-                const bool inside = SUM != WS_NONE && unit &&
-                                    __all(lo + to >= A.t0 && hi + to <= A.tmax);
-                if (inside)
-                    sweep(std::integral_constant<int, SUM == WS_NONE ? 1 : 2>());
-                else if (unit)
-                    sweep(std::integral_constant<int, 1>());
-                else
-                    sweep(std::integral_constant<int, 0>());
-            }
-            if (SUM == WS_NONE) continue;
-            if (!GEOM && unit) {
-#pragma unroll
-                for (int f = 0; f < FC; ++f) part[f] *= (to == to) ? wo : 0.0f;
-            }
-            if (SUM == WS_BOTH) {
-#pragma unroll
-                for (int f = 0; f < FC; ++f) acc[f] += part[f];
-            } else if (act) {
-#pragma unroll
-                for (int f = 0; f < FC; ++f)
-                    if (f < nf) {
-                        float *q = A.out + ((int64_t)(f0 + f) * no + o) * A.np + p;
-                        *q = (i0 == 0) ? part[f] : *q + part[f];
-                    }
-            }
-        }
-    }
+    wave_sweep<GK, SUM, FC, GEOM, MODE>(A, W, sm, share, nw, wave, lane, act, p, pv, f0, nf, acc);
     if (SUM == WS_BOTH) {
         __syncthreads();
 #pragma unroll

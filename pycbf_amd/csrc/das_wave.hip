@@ -18,10 +18,9 @@ int wave_launch_sample(int gk, const DasArgs &a, const WaveArgs &w, int sum, int
 
 bool das_wave_applies(int gk, const DasArgs &a)
 {
-    if (a.nsrc > WAVE_MAX_NSRC || (gk == GK_LINEAR && a.nsrc < 2)) return false;
+    if (gk == GK_LINEAR && a.nsrc < 2) return false;      // reads pairs
+    if (gk == GK_NEAREST && a.nsrc > 1 << 22) return false;  // nsrc - 1/2 as a float
     if (a.np > (int64_t)1 << 28) return false;  // 16 threads per pixel within a 32-bit grid
-    // the last sample time must select a knot of the trace
-    if (gk != GK_NEAREST && !((int)((a.tmax - a.t0) / a.dt) <= a.nsrc - 1)) return false;
     // the cubic over 4 or more frames is staged in LDS (k_das_cubic_dma)
     return gk != GK_CUBIC || a.nfr < 4;
 }
@@ -85,9 +84,7 @@ int launch_das_wave(int gk, const DasArgs &a0, int max_part, float *partial, int
                     : a.sumflag == PYCBF_SUM_NONE    ? WS_NONE
                                                      : WS_SEP;
     const int fc = a.nfr >= 4 ? 4 : (a.nfr >= 2 ? 2 : 1);
-    int mode = WM_DIV;
-    if (a.rdt == 1.0f / a.dt && recip_division_exact(a.dt))
-        mode = a.t0 == 0.0f ? WM_RECIP0 : WM_RECIP;
+    const int mode = wave_mode_of(a.t0, a.dt, a.rdt, a.tmax, a.nsrc);
     w.weights = !(a.geo && a.thresh > 0.0f && a.thresh <= 1.0f);
     const int64_t ntiles = (a.np + 63) / 64;
     const int64_t passes = (a.nfr + fc - 1) / fc;
@@ -129,9 +126,7 @@ int launch_das_wave(int gk, const DasArgs &a0, int max_part, float *partial, int
     }
     float *final_out = a.out;
     if (sum == WS_BOTH && nchunk > 1) a.out = partial;
-    const size_t lds = std::max((size_t)w.ib * 64 * 4 * (w.weights ? 2 : 1) + (size_t)w.ib * 4 +
-                                    (size_t)nw * 128 * 4,
-                                (size_t)nw * fc * 64 * 4);
+    const size_t lds = std::max(wave_lds_bytes(w.ib, w.weights, nw), (size_t)nw * fc * 64 * 4);
     const dim3 grid((unsigned)(w.slab ? ntiles * 8 : ntiles), (unsigned)(w.slab ? 1 : nchunk),
                     (unsigned)passes);
     int rc;

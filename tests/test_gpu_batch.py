@@ -123,3 +123,35 @@ def test_autotune_then_graph_replays(setup):
             ok = ~torch.isnan(e)
             assert float((o[ok] - e[ok]).abs().max()) <= 1e-5 * float(e[ok].abs().max() + 1e-30), (k, r)
     _check(batch, reqs, refs)
+
+
+@pytest.mark.parametrize("t0", [0.0, 1.5e-6])
+@pytest.mark.parametrize("thresh", [0.0, 1e-2, 1.5])
+def test_batch_gather_branches(t0, thresh):
+    """Few transmits (the waves split the receive elements), more transmits than
+    one LDS block, grids smaller than a patch and with ragged edges, thresholds
+    where zero weights count (0) and where nothing does (1.5), and a trace
+    start away from zero, against the single-request beamformer (1e-5 of the
+    peak, summation order)."""
+    import torch
+    from pycbf_amd import sim
+    from pycbf_amd.gpu import SyntheticBeamformer
+    from pycbf_amd.gpu.batch import BatchRequest, RaggedBatch
+    nt, dt = 500, 1.0 / sim.FS
+    rng = np.random.default_rng(3)
+    reqs, singles = [], []
+    for ntx, nrx, nx, nz in ((1, 20, 5, 7), (7, 130, 9, 17), (8, 9, 33, 8), (170, 3, 16, 21)):
+        xele = sim.linear_array(nrx)
+        _, _, pnts = sim.grid(nx, nz, (-2e-3, 2e-3), (2e-3, 7e-3))
+        p = sim.pw_synthetic(np.radians(np.linspace(-9, 9, ntx)) if ntx > 1 else np.zeros(1), xele, pnts)
+        reqs.append(BatchRequest(params=p, gridshape=(nx, nz), thresh=thresh))
+        singles.append(SyntheticBeamformer(**p, t0=t0, dt=dt, nt=nt, interp={"kind": "cubic"}, thresh=thresh))
+    batch = RaggedBatch(reqs, nt=nt, dt=dt, t0=t0)
+    for v in batch.rf_views:
+        v.copy_(torch.as_tensor(rng.standard_normal(tuple(v.shape)).astype(np.float32)))
+    for tile, rchunk in ((8, 16), (16, 128), (32, 32)):
+        batch.configure(tile, rchunk)
+        batch.run()
+        for bf, v, o in zip(singles, batch.rf_views, batch.outputs):
+            ref = bf(v, out_as_numpy=False).reshape(o.shape)
+            assert float((o - ref).abs().max()) <= 1e-5 * float(ref.abs().max()), (tile, rchunk, tuple(o.shape))
