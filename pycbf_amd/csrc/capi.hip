@@ -659,6 +659,7 @@ int pycbf_debug_indices(const pycbf_rfinfo *info, const float *tautx, const floa
 struct BwdPlan {
     size_t bounds = 0, coef = 0, uscr = 0, gy = 0, ge = 0, gc2 = 0, gc3 = 0, mbits = 256;
     size_t y2 = 0, up = 0, gu = 0;  // nearest, usf > 1
+    size_t tau = 0;                 // delays of the synthetic geometry
     size_t gc0 = 0;                 // partial sums of d loss / d c0 (synthetic geometry)
     size_t total = 0;
 };
@@ -669,7 +670,13 @@ static BwdPlan plan_bwd(const pycbf_rfinfo *info, int64_t nfr, int64_t np, int k
     const int64_t nt = info->tinfo.nx;
     const int64_t nch = nfr * info->ntx * info->nrx;
     b.bounds = align_up((size_t)das_tiles(np) * (size_t)(info->ntx + info->nrx) * 2 * 4, 256);
-    b.gc0 = align_up((size_t)das_tiles(np) * (size_t)(info->ntx + info->nrx) * 8, 256);
+    // a double per (tile of 256, element), or up to 8 per 64 pixels and axis
+    b.gc0 = align_up((size_t)das_tiles(np) * (size_t)(info->ntx + info->nrx + 64) * 8, 256);
+    // Synthetic geometry, channel-data gradient: its delays as a table while that
+    // is small (every channel reads two rows of it; beyond 256 MB the kernels
+    // evaluate the geometry again for each channel)
+    const size_t tau = align_up((size_t)np * (size_t)(info->ntx + info->nrx) * 4, 256);
+    if (info->ndim >= 2 && nt <= 4096 && tau <= (size_t)256 << 20) b.tau = tau;
     if (kind == PYCBF_INTERP_CUBIC) {
         b.coef = align_up((size_t)nch * (size_t)(nt + 1) * 8, 256);
         b.uscr = spline_scratch_bytes(nch, (int32_t)nt);
@@ -686,7 +693,7 @@ static BwdPlan plan_bwd(const pycbf_rfinfo *info, int64_t nfr, int64_t np, int k
         b.gy = b.ge = align_up((size_t)nch * (size_t)(nt + 1) * 4, 256);
     }
     b.total = b.bounds + b.coef + b.uscr + b.gy + b.ge + b.gc2 + b.gc3 + b.mbits + b.y2 + b.up +
-              b.gu + b.gc0 + 12 * 256;
+              b.gu + b.gc0 + b.tau + 12 * 256;
     return b;
 }
 
@@ -757,13 +764,24 @@ static int bwd_run(const pycbf_rfinfo *info, const float *rf, int64_t nfr, int64
     b.bounds = bounds;
     b.mbits = (unsigned *)cv.take(plan.mbits);
     b.gc0part = (double *)cv.take(plan.gc0);
+    // the channel-data gradient does not depend on the channel data: their
+    // table is built only for the gradients of delays, weights or c0
+    const bool elems = gtautx || gapodtx || gtaurx || gapodrx || gc0;
+    if (elems && np >= 4096) {
+        b.fast = (int *)b.mbits + 8;
+        const float *row = b.nrx >= 2 ? b.trx : b.ttx;
+        const int64_t last = (b.nrx >= 2 ? b.nrx : b.ntx) - 1;
+        if ((rc = b.geo ? launch_fast_axis(b.pvec, b.pvec + b.geo - 1, b.geo, np, b.fast, s)
+                        : launch_fast_axis(row, row + last * np, 1, np, b.fast, s)))
+            return rc;
+    }
     if (interp_kind == PYCBF_INTERP_CUBIC) {
         float2 *coef = (float2 *)cv.take(plan.coef);
         float *u = (float *)cv.take(plan.uscr);
         b.gy = (float *)cv.take(plan.gy);
         b.ge = (float *)cv.take(plan.ge);
         b.gstride = nt + 1;
-        if ((rc = launch_spline_coefs(rf, nch, nt, dt, u, coef, s))) return rc;
+        if (elems && (rc = launch_spline_coefs(rf, nch, nt, dt, u, coef, s))) return rc;
         b.src = (const float *)coef;
     } else if (interp_kind == PYCBF_INTERP_KORDER_CUBIC) {
         float4 *coef = (float4 *)cv.take(plan.coef);
@@ -774,7 +792,7 @@ static int bwd_run(const pycbf_rfinfo *info, const float *rf, int64_t nfr, int64
         b.gstride = nt;
         b.S = S;
         b.k = param;
-        if ((rc = launch_korder_coefs(rf, nch, nt, S, param, coef, s))) return rc;
+        if (elems && (rc = launch_korder_coefs(rf, nch, nt, S, param, coef, s))) return rc;
         b.src = (const float *)coef;
     } else if (interp_kind == PYCBF_INTERP_AKIMA || interp_kind == PYCBF_INTERP_MAKIMA) {
         float4 *coef = (float4 *)cv.take(plan.coef);
@@ -785,15 +803,15 @@ static int bwd_run(const pycbf_rfinfo *info, const float *rf, int64_t nfr, int64
         b.gstride = nt;
         b.rf = rf;
         b.modified = interp_kind == PYCBF_INTERP_MAKIMA;
-        if ((rc = launch_akima_coefs(rf, nch, nt, b.modified, coef, s))) return rc;
+        if (elems && (rc = launch_akima_coefs(rf, nch, nt, b.modified, coef, s))) return rc;
         b.src = (const float *)coef;
     } else if (interp_kind == PYCBF_INTERP_NEAREST && param > 1) {
         // nearest on the upsampled trace, as the forward gathers it
         float *y2 = (float *)cv.take(plan.y2);
         float *u = (float *)cv.take(plan.uscr);
         float *up = (float *)cv.take(plan.up);
-        if ((rc = launch_spline_y2(rf, nch, nt, dt, u, y2, s))) return rc;
-        if ((rc = launch_upsample(rf, y2, nch, nt, t0, dt, param, up, s))) return rc;
+        if (elems && (rc = launch_spline_y2(rf, nch, nt, dt, u, y2, s))) return rc;
+        if (elems && (rc = launch_upsample(rf, y2, nch, nt, t0, dt, param, up, s))) return rc;
         const int ntu = param * (nt - 1) + 1;
         b.src = up;
         b.nt = ntu;
@@ -806,19 +824,27 @@ static int bwd_run(const pycbf_rfinfo *info, const float *rf, int64_t nfr, int64
         b.gy = grf;
         b.gstride = nt;
     }
-    if (grf) {
-        tb.np = np;
-        tb.ntx = b.ntx;
-        tb.nrx = b.nrx;
-        tb.thresh = thresh;
-        tb.perm = nullptr;
-        if ((rc = launch_tile_bounds(tb, bounds, s))) return rc;
-    }
     const int gk = interp_kind == PYCBF_INTERP_NEAREST  ? GK_NEAREST
                    : interp_kind == PYCBF_INTERP_LINEAR ? GK_LINEAR
                    : interp_kind == PYCBF_INTERP_CUBIC  ? GK_CUBIC
                    : interp_kind == PYCBF_INTERP_KORDER_CUBIC ? GK_KORDER
                                                               : GK_AKIMA;
+    if (grf) {
+        if (plan.tau && b.geo && thresh > 0.0f && thresh <= 1.0f)
+            b.unit_tau = (float *)cv.take(plan.tau);
+        bool per_channel = false;
+        if ((rc = bwd_per_channel(gk, b, per_channel))) return rc;
+        // the delay ranges serve the transposed gather per pixel tile, and the one
+        // per channel where it evaluates the geometry itself
+        if (!per_channel || (b.geo && !b.unit_tau)) {
+            tb.np = np;
+            tb.ntx = b.ntx;
+            tb.nrx = b.nrx;
+            tb.thresh = thresh;
+            tb.perm = nullptr;
+            if ((rc = launch_tile_bounds(tb, bounds, s))) return rc;
+        }
+    }
     if ((rc = launch_das_bwd(gk, b, gtautx, gapodtx, gtaurx, gapodrx, grf, gc0, s))) return rc;
     if (grf && interp_kind == PYCBF_INTERP_NEAREST && param > 1) {
         float *gy = (float *)cv.take(plan.gy);

@@ -170,11 +170,24 @@ struct BwdArgs {
     float c0, rc0;  // rc0 = 1 / c0 rounded
     double *gc0part;  // per-workgroup partial sums of d loss / d c0 (geo > 0), or null
     int gc0_off;      // first partial of this launch
+    float *unit_tau;  // scratch for (ntx + nrx, np) delays (geo > 0, thresh in (0, 1]), or null
+    int *fast;        // the pixels' fast axis (launch_fast_axis), or null
 };
+// Whether the channel-data gradient runs one workgroup per channel (the whole
+// trace's bins in LDS); else per pixel tile, which reads a.bounds.
+int bwd_per_channel(int gk, const BwdArgs &a, bool &yes);
 // gc0 (geo > 0, may be null): d loss / d c0, one float, reduced in a fixed order
 // from a.gc0part ((ntx + nrx) * das_tiles(np) doubles)
 int launch_das_bwd(int gk, const BwdArgs &a, float *gtautx, float *gapodtx, float *gtaurx,
                    float *gapodrx, float *grf, float *gc0, hipStream_t s);
+// Delay / apodisation gradients (and c0 partials) of one axis on wave tiles
+// (das_bwd_elem.hip): 0 when launched, with the number of c0 partials in
+// `parts`; 1 when the call is not one it takes; another status on failure.
+int launch_bwd_elem(int gk, const BwdArgs &a, int outer_tx, int &parts, hipStream_t s);
+// Writes to *fast (device) the length of the pixel grid's fast axis, read off
+// two rows (delays, or coordinates `stride` floats apart), 0 when they show none.
+int launch_fast_axis(const float *row0, const float *row1, int stride, int64_t np, int *fast,
+                     hipStream_t s);
 // nearest with usf > 1: cotangents gu of the upsampled trace (nch, usf (nt-1)
 // + 1) -> spline-table cotangents gy, ge (nch, nt + 1) -> grf (nch, nt)
 int launch_upsample_adjoint(const float *gu, int64_t nch, int32_t nt, int32_t usf, float t0,

@@ -35,6 +35,7 @@
 #include <math.h>
 
 #include <algorithm>
+#include <type_traits>
 
 #include "common.h"
 #include "das_dev.h"
@@ -480,6 +481,22 @@ __global__ __launch_bounds__(256) void k_das_bwd_rf(BwdArgs A)
     }
 }
 
+// Delays of the synthetic geometry with NaN where the element's weight is zero
+// (thresh in (0, 1]: such a sample never counts, and every other weight is 1):
+// tau[e][p], transmits first.
+template <int GEO, bool FD>
+__global__ __launch_bounds__(256) void k_unit_delays(BwdArgs A, float *__restrict__ tau)
+{
+    const int64_t p = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (p >= A.np) return;
+    const int e = blockIdx.y;
+    float pv[3];
+    bwd_pixel<GEO>(A, p, pv);
+    float t, ap;
+    bwd_elem<GEO, FD>(A, e < A.ntx, e < A.ntx ? e : e - A.ntx, p, pv, t, ap);
+    tau[(int64_t)e * A.np + p] = ap != 0.0f ? t : NAN;
+}
+
 // Transposed gather with one workgroup per channel (frame, transmit,
 // receive) for traces of up to 4096 samples: the workgroup sweeps every pixel
 // of the channel into fixed-point LDS bins covering the whole trace (y and,
@@ -487,17 +504,24 @@ __global__ __launch_bounds__(256) void k_das_bwd_rf(BwdArgs A)
 // cotangent rows once with plain stores.  No global atomics, no zero fill of
 // the rows beforehand, and the integer sums make the result independent of
 // the order of the pixels.  16 waves per workgroup sweep 1024 pixels per
-// step; a wave skips its 64 pixels when the tile's delay range leaves the
-// channel unused.
-template <int GK, int GEO, bool FD>
+// step.  SRC: where delays and weights come from.
+//   RF_TABLES  the tables; the delays are read only where the weight passes
+//   RF_UNIT    k_unit_delays' table (a NaN delay: no sample)
+//   RF_GEOM    the geometry in registers; a wave skips its 64 pixels when the
+//              tile's delay range leaves the channel unused
+// A contribution becomes an integer by adding 1.5 2^52 to it in double, exact to
+// the last bit kept while it stays below 2^51 (MAGIC; two instructions and an
+// integer subtraction, against about ten for the conversion): images of 256
+// pixels and more, whose bins leave that much room.
+// 31 x 128 x 4096 onto 256 x 256, cubic, tables: 606 -> 433 us; 16 x 64 x
+// 2048 onto 192 x 256, linear, geometry: 222 -> 74 us and 11 for its table.
+enum RfSource { RF_TABLES = 0, RF_UNIT = 1, RF_GEOM = 2 };
+
+template <int GK, int GEO, bool FD, int SRC, bool MAGIC>
 __global__ __launch_bounds__(1024) void k_das_bwd_rf_ch(BwdArgs A)
 {
     extern __shared__ unsigned long long bins[];
     const int nb = A.gstride;  // bins per array: the row length
-    unsigned long long *by = bins;
-    unsigned long long *be = bins + nb;  // cubic only
-    float *byf = reinterpret_cast<float *>(by);
-    float *bef = reinterpret_cast<float *>(be);
     const int tid = threadIdx.x;
     const int64_t chan = blockIdx.x;
     const int rx = (int)(chan % A.nrx);
@@ -509,98 +533,118 @@ __global__ __launch_bounds__(1024) void k_das_bwd_rf_ch(BwdArgs A)
     const double scale = bwd_scale(A.mbits, per_bin);
     const bool fix = scale > 0.0;  // uniform
     const double iscale = fix ? 1.0 / scale : 0.0;
-    auto bin_add = [&](unsigned long long *b, float *bf, int i, float v) {
-        if (fix)
-            atomicAdd(b + i, (unsigned long long)(long long)((double)v * scale));
-        else
-            atomicAdd(bf + i, v);
-    };
     constexpr bool HERM = GK == GK_KORDER || GK == GK_AKIMA;
-    unsigned long long *b2 = bins + 2 * nb, *b3 = bins + 3 * nb;  // Hermite kinds only
-    float *b2f = reinterpret_cast<float *>(b2), *b3f = reinterpret_cast<float *>(b3);
     const int narr = GK == GK_CUBIC ? 2 : (HERM ? 4 : 1);
     for (int t = tid; t < narr * nb; t += blockDim.x) bins[t] = 0ull;
     __syncthreads();
 
-    for (int64_t base = 0; base < A.np; base += blockDim.x) {
-        const int64_t p = base + tid;
-        // the wave's pixels lie in one tile of 256: skip it when the tile's
-        // delay range selects no sample of this channel (wave-uniform)
-        const int64_t tile = (base + (tid & ~63)) >> 8;
-        if ((base + (tid & ~63)) >= A.np) continue;
-        const float *bt = A.bounds + (tile * nent + tx) * 2;
-        const float *br = A.bounds + (tile * nent + A.ntx + rx) * 2;
-        const float xlo = bt[0] + br[0], xhi = bt[1] + br[1];
-        if (!(xlo <= xhi)) continue;
-        if (p >= A.np) continue;
-        float ttx = 0.0f, atx = 0.0f, trx = 0.0f, arx = 0.0f;
-        if (GEO == 0) {
-            // tables: the delays are read only where the weight passes
-            atx = A.atx[(int64_t)tx * A.np + p];
-            arx = A.arx[(int64_t)rx * A.np + p];
-        } else {
-            float pv[3];
-            bwd_pixel<GEO>(A, p, pv);
-            bwd_elem<GEO, FD>(A, true, tx, p, pv, ttx, atx);
-            bwd_elem<GEO, FD>(A, false, rx, p, pv, trx, arx);
-        }
-        const float w = atx * arx;
-        if (!(fabsf(w) >= A.thresh)) continue;
-        if (GEO == 0) {
-            ttx = A.ttx[(int64_t)tx * A.np + p];
-            trx = A.trx[(int64_t)rx * A.np + p];
-        }
-        const float x = ttx + trx;
-        const float g = A.gout[gout_index(A.sumflag, f, tx, rx, A.ntx, A.nrx, A.np, p)] * w;
-        if (g == 0.0f) continue;
-        if (GK == GK_NEAREST) {
-            int it = 0;
-            if (nearest_index(x, A.t0, A.dt, A.nt, it)) bin_add(by, byf, it, g);
-        } else if (HERM) {
-            int j = 0;
-            if (!knot_at<FD>(A, x, j)) continue;
-            // |t| <= 1 (to rounding): every contribution stays within the bound
-            const float t = (GK == GK_KORDER) ? ((x - A.t0) - A.dt * (float)j) * A.rdt
-                                              : (x - (A.t0 + A.dt * (float)j)) * A.rdt;
-            bin_add(by, byf, j, g);
-            bin_add(be, bef, j, g * t);
-            bin_add(b2, b2f, j, g * (t * t));
-            bin_add(b3, b3f, j, g * ((t * t) * t));
-        } else {
-            int j = 0;
-            if (!knot_at<FD>(A, x, j)) continue;
-            const float xlead = A.t0 + A.dt * (float)(j + 1);
-            const float xlag = A.t0 + A.dt * (float)j;
-            float a, b;
-            if (GK == GK_LINEAR) {
-                a = (xlead - x) / A.dt;
-                b = (x - xlag) / A.dt;
+    // rows of this channel's elements, by 32-bit pixel offsets
+    const float *r_atx = SRC == RF_TABLES ? A.atx + (int64_t)tx * A.np : nullptr;
+    const float *r_arx = SRC == RF_TABLES ? A.arx + (int64_t)rx * A.np : nullptr;
+    const float *r_ttx = SRC != RF_GEOM ? A.ttx + (int64_t)tx * A.np : nullptr;
+    const float *r_trx = SRC != RF_GEOM ? A.trx + (int64_t)rx * A.np : nullptr;
+    const float *r_g = A.gout + gout_index(A.sumflag, f, tx, rx, A.ntx, A.nrx, A.np, 0);
+    auto sweep = [&](auto fixc) {
+        constexpr bool FIX = decltype(fixc)::value;
+        auto bin_add = [&](int arr, int i, float v) {
+            const int at = arr * nb + i;
+            if (!FIX) {
+                atomicAdd(reinterpret_cast<float *>(bins + arr * nb) + i, v);
+            } else if (MAGIC) {
+                const double m = __builtin_fma((double)v, scale, 0x1.8p+52);
+                atomicAdd(bins + at, (unsigned long long)__double_as_longlong(m) -
+                                         0x4338000000000000ull);
             } else {
-                a = (xlead - x) * A.rdt;
-                b = (x - xlag) * A.rdt;
+                atomicAdd(bins + at, (unsigned long long)(long long)((double)v * scale));
             }
-            // sample j+1 exists for the cubic table (zero entry at nt); for
-            // linear the forward reads 0 past the last sample
-            bin_add(by, byf, j, g * a);
-            if (GK == GK_CUBIC || j + 1 < A.nt) bin_add(by, byf, j + 1, g * b);
-            if (GK == GK_CUBIC) {
-                bin_add(be, bef, j, g * __builtin_fmaf(a * a, a, -a));
-                bin_add(be, bef, j + 1, g * __builtin_fmaf(b * b, b, -b));
+        };
+        for (int64_t base = 0; base < A.np; base += blockDim.x) {
+            const int64_t p64 = base + tid;
+            if (SRC == RF_GEOM) {
+                // the wave's pixels lie in one tile of 256 (wave-uniform)
+                const int64_t tile = (base + (tid & ~63)) >> 8;
+                if ((base + (tid & ~63)) >= A.np) continue;
+                const float *bt = A.bounds + (tile * nent + tx) * 2;
+                const float *br = A.bounds + (tile * nent + A.ntx + rx) * 2;
+                if (!(bt[0] + br[0] <= bt[1] + br[1])) continue;
+            }
+            if (p64 >= A.np) continue;
+            const uint32_t p = (uint32_t)p64;
+            float ttx = 0.0f, trx = 0.0f, w = 1.0f;
+            if (SRC == RF_TABLES) {
+                w = r_atx[p] * r_arx[p];
+                if (!(fabsf(w) >= A.thresh)) continue;
+                ttx = r_ttx[p];
+                trx = r_trx[p];
+            } else if (SRC == RF_UNIT) {
+                ttx = r_ttx[p];
+                trx = r_trx[p];
+            } else {
+                float pv[3], atx, arx;
+                bwd_pixel<GEO>(A, p, pv);
+                bwd_elem<GEO, FD>(A, true, tx, p, pv, ttx, atx);
+                bwd_elem<GEO, FD>(A, false, rx, p, pv, trx, arx);
+                w = atx * arx;
+                if (!(fabsf(w) >= A.thresh)) continue;
+            }
+            const float x = ttx + trx;
+            int j = 0;
+            if (GK == GK_NEAREST) {
+                if (!nearest_index(x, A.t0, A.dt, A.nt, j)) continue;
+            } else {
+                if (!knot_at<FD>(A, x, j)) continue;
+            }
+            const float g = r_g[p] * w;
+            if (g == 0.0f) continue;
+            if (GK == GK_NEAREST) {
+                bin_add(0, j, g);
+            } else if (HERM) {
+                // |t| <= 1 (to rounding): every contribution stays within the bound
+                const float t = (GK == GK_KORDER) ? ((x - A.t0) - A.dt * (float)j) * A.rdt
+                                                  : (x - (A.t0 + A.dt * (float)j)) * A.rdt;
+                bin_add(0, j, g);
+                bin_add(1, j, g * t);
+                bin_add(2, j, g * (t * t));
+                bin_add(3, j, g * ((t * t) * t));
+            } else {
+                const float xlead = A.t0 + A.dt * (float)(j + 1);
+                const float xlag = A.t0 + A.dt * (float)j;
+                float a, b;
+                if (GK == GK_LINEAR) {
+                    a = FD ? div_rn(xlead - x, A.dt, A.rdt) : (xlead - x) / A.dt;
+                    b = FD ? div_rn(x - xlag, A.dt, A.rdt) : (x - xlag) / A.dt;
+                } else {
+                    a = (xlead - x) * A.rdt;
+                    b = (x - xlag) * A.rdt;
+                }
+                // sample j+1 exists for the cubic table (zero entry at nt); for
+                // linear the forward reads 0 past the last sample
+                bin_add(0, j, g * a);
+                if (GK == GK_CUBIC || j + 1 < A.nt) bin_add(0, j + 1, g * b);
+                if (GK == GK_CUBIC) {
+                    bin_add(1, j, g * __builtin_fmaf(a * a, a, -a));
+                    bin_add(1, j + 1, g * __builtin_fmaf(b * b, b, -b));
+                }
             }
         }
-    }
+    };
+    if (fix)
+        sweep(std::true_type());
+    else
+        sweep(std::false_type());  // a bound is not finite: float bins
     __syncthreads();
     float *gy = A.gy + chan * A.gstride;
     float *ge = GK != GK_NEAREST && GK != GK_LINEAR ? A.ge + chan * A.gstride : nullptr;
-    auto take = [&](const unsigned long long *b, const float *bf, int t) -> float {
-        return fix ? (float)((double)(long long)b[t] * iscale) : bf[t];
+    auto take = [&](int arr, int t) -> float {
+        return fix ? (float)((double)(long long)bins[arr * nb + t] * iscale)
+                   : reinterpret_cast<const float *>(bins + arr * nb)[t];
     };
     for (int t = tid; t < nb; t += blockDim.x) {
-        gy[t] = take(by, byf, t);
-        if (GK == GK_CUBIC || HERM) ge[t] = take(be, bef, t);
+        gy[t] = take(0, t);
+        if (GK == GK_CUBIC || HERM) ge[t] = take(1, t);
         if (HERM) {
-            A.gc2[chan * A.gstride + t] = take(b2, b2f, t);
-            A.gc3[chan * A.gstride + t] = take(b3, b3f, t);
+            A.gc2[chan * A.gstride + t] = take(2, t);
+            A.gc3[chan * A.gstride + t] = take(3, t);
         }
     }
 }
@@ -1103,51 +1147,103 @@ static int fill_zero(float *p, int64_t n, hipStream_t s)
     return check_launch("fill zero");
 }
 
+static int bwd_arrays(int gk)
+{
+    return gk == GK_CUBIC ? 2 : (gk == GK_KORDER || gk == GK_AKIMA ? 4 : 1);
+}
+
+int bwd_per_channel(int gk, const BwdArgs &a, bool &yes)
+{
+    int dev = 0, max_lds = 0;
+    if (int rc = check(hipGetDevice(&dev), "device")) return rc;
+    if (int rc = check(hipDeviceGetAttribute(&max_lds, hipDeviceAttributeMaxSharedMemoryPerBlock,
+                                             dev),
+                       "LDS per workgroup"))
+        return rc;
+    yes = a.gstride <= 4097 && (size_t)bwd_arrays(gk) * a.gstride * 8 <= (size_t)max_lds &&
+          (int64_t)a.nfr * a.ntx * a.nrx <= 0x7fffffff && a.np <= 0x7fffffff;
+    return 0;
+}
+
+template <int GK, int GEO, bool FD, int SRC>
+static int launch_rf_ch_src(const BwdArgs &a, int64_t nch, size_t lds, hipStream_t s)
+{
+    // the magic conversion needs contributions below 2^51: bwd_scale leaves them
+    // below 2^(60 - per_bin), per_bin >= 10
+    if (a.np >= 256)
+        hipLaunchKernelGGL((k_das_bwd_rf_ch<GK, GEO, FD, SRC, true>), dim3((unsigned)nch),
+                           dim3(1024), lds, s, a);
+    else
+        hipLaunchKernelGGL((k_das_bwd_rf_ch<GK, GEO, FD, SRC, false>), dim3((unsigned)nch),
+                           dim3(1024), lds, s, a);
+    return check_launch("das_bwd_rf");
+}
+
+template <int GK, int GEO, bool FD>
+static int launch_rf_ch(const BwdArgs &a, int64_t nch, size_t lds, hipStream_t s)
+{
+    if constexpr (GEO == 0) {
+        return launch_rf_ch_src<GK, GEO, FD, RF_TABLES>(a, nch, lds, s);
+    } else {
+        if (a.unit_tau) {
+            BwdArgs b = a;
+            b.ttx = a.unit_tau;
+            b.trx = a.unit_tau + (int64_t)a.ntx * a.np;
+            hipLaunchKernelGGL((k_unit_delays<GEO, FD>),
+                               dim3((unsigned)((a.np + 255) / 256), a.ntx + a.nrx), dim3(256), 0, s,
+                               b, a.unit_tau);
+            if (int rc = check_launch("unit delays")) return rc;
+            return launch_rf_ch_src<GK, GEO, FD, RF_UNIT>(b, nch, lds, s);
+        }
+        return launch_rf_ch_src<GK, GEO, FD, RF_GEOM>(a, nch, lds, s);
+    }
+}
+
 template <int GK, int GEO, bool FD>
 static int launch_bwd_t(const BwdArgs &a, float *gtautx, float *gapodtx, float *gtaurx,
                         float *gapodrx, float *grf, float *gc0, hipStream_t s)
 {
     const unsigned ptiles = (unsigned)((a.np + 255) / 256);
     const bool want_c0 = GEO > 0 && gc0 && a.gc0part;
-    if (gtautx || gapodtx || want_c0) {
+    int64_t nparts = 0;
+    auto elements = [&](int outer_tx, float *gtau, float *gapod) {
         BwdArgs b = a;
-        b.gtau = gtautx;
-        b.gapod = gapodtx;
+        b.gtau = gtau;
+        b.gapod = gapod;
         b.gc0part = want_c0 ? a.gc0part : nullptr;
-        b.gc0_off = 0;
+        b.gc0_off = (int)nparts;
         ProfScope ps("das_bwd_tau", s);
-        hipLaunchKernelGGL((k_das_bwd_tau<GK, 1, GEO, FD>), dim3(ptiles, a.ntx), dim3(256), 0, s, b);
-        if (int rc = check_launch("das_bwd_tau")) return rc;
-    }
-    if (gtaurx || gapodrx || want_c0) {
-        BwdArgs b = a;
-        b.gtau = gtaurx;
-        b.gapod = gapodrx;
-        b.gc0part = want_c0 ? a.gc0part : nullptr;
-        b.gc0_off = (int)(ptiles * (unsigned)a.ntx);
-        ProfScope ps("das_bwd_tau", s);
-        hipLaunchKernelGGL((k_das_bwd_tau<GK, 0, GEO, FD>), dim3(ptiles, a.nrx), dim3(256), 0, s, b);
-        if (int rc = check_launch("das_bwd_tau")) return rc;
-    }
+        int parts = 0;
+        int rc = launch_bwd_elem(GK, b, outer_tx, parts, s);
+        if (rc == 1) {
+            // one lane per (element, pixel): c0 alone over an axis too long for
+            // LDS, one-sample traces
+            const dim3 grid(ptiles, outer_tx ? a.ntx : a.nrx);
+            if (outer_tx)
+                hipLaunchKernelGGL((k_das_bwd_tau<GK, 1, GEO, FD>), grid, dim3(256), 0, s, b);
+            else
+                hipLaunchKernelGGL((k_das_bwd_tau<GK, 0, GEO, FD>), grid, dim3(256), 0, s, b);
+            parts = (int)(grid.x * grid.y);
+            rc = check_launch("das_bwd_tau");
+        }
+        nparts += parts;
+        return rc;
+    };
+    if (gtautx || gapodtx || want_c0)
+        if (int rc = elements(1, gtautx, gapodtx)) return rc;
+    if (gtaurx || gapodrx || want_c0)
+        if (int rc = elements(0, gtaurx, gapodrx)) return rc;
     if (want_c0) {
-        hipLaunchKernelGGL(k_gc0_sum, dim3(1), dim3(256), 0, s, (const double *)a.gc0part,
-                           (int64_t)ptiles * (a.ntx + a.nrx), gc0);
+        hipLaunchKernelGGL(k_gc0_sum, dim3(1), dim3(256), 0, s, (const double *)a.gc0part, nparts,
+                           gc0);
         if (int rc = check_launch("gc0_sum")) return rc;
     }
     if (grf) {
         const int64_t nch = (int64_t)a.nfr * a.ntx * a.nrx;
         ProfScope ps("das_bwd_rf", s);
-        // one workgroup per channel while the whole trace's bins fit in LDS
-        const size_t ch_lds =
-            (size_t)(GK == GK_CUBIC ? 2 : (GK == GK_KORDER || GK == GK_AKIMA ? 4 : 1)) *
-            a.gstride * 8;
-        int dev = 0, max_lds = 0;
-        if (int rc = check(hipGetDevice(&dev), "device")) return rc;
-        if (int rc = check(hipDeviceGetAttribute(&max_lds, hipDeviceAttributeMaxSharedMemoryPerBlock,
-                                                 dev),
-                           "LDS per workgroup"))
-            return rc;
-        const bool per_channel = a.gstride <= 4097 && ch_lds <= (size_t)max_lds && nch <= 0x7fffffff;
+        bool per_channel = false;
+        if (int rc = bwd_per_channel(GK, a, per_channel)) return rc;
+        const size_t ch_lds = (size_t)bwd_arrays(GK) * a.gstride * 8;
         // bound of the contributions for the fixed-point bins
         if (int rc = fill_zero(reinterpret_cast<float *>(a.mbits), 3, s)) return rc;
         int64_t ngout = (int64_t)a.nfr * a.np;
@@ -1159,8 +1255,7 @@ static int launch_bwd_t(const BwdArgs &a, float *gtautx, float *gapodtx, float *
         hipLaunchKernelGGL(k_bwd_scale, dim3(sb, 3), dim3(256), 0, s, a, ngout);
         if (int rc = check_launch("das_bwd_scale")) return rc;
         if (per_channel) {
-            hipLaunchKernelGGL((k_das_bwd_rf_ch<GK, GEO, FD>), dim3((unsigned)nch), dim3(1024), ch_lds, s,
-                               a);
+            if (int rc = launch_rf_ch<GK, GEO, FD>(a, nch, ch_lds, s)) return rc;
         } else {
             if (GK == GK_CUBIC || GK == GK_KORDER || GK == GK_AKIMA) {
                 if (int rc = fill_zero(a.gy, nch * a.gstride, s)) return rc;

@@ -25,28 +25,41 @@ bool das_wave_applies(int gk, const DasArgs &a)
     return gk != GK_CUBIC || a.nfr < 4;
 }
 
-// Length of the pixel grid's fast axis, read off two delay rows: along a line
+// Length of the pixel grid's fast axis, read off two rows of delays (or of one
+// coordinate, `stride` floats apart): along a line
 // of pixels the delay to an element outside the line's span changes in one
 // direction, and turns back where the next line starts.  The first turn of
 // either row that divides the pixel count evenly is taken (the longer of the
 // two, 0 when neither does).  Only the grouping of pixels into tiles depends
 // on it, never a result.
-constexpr int FAST_MIN = 32, FAST_MAX = 8192;
+constexpr int FAST_MIN = 32, FAST_MAX = 4096;
 
 __global__ __launch_bounds__(1024) void k_fast_axis(const float *__restrict__ row0,
-                                                    const float *__restrict__ row1, int64_t np,
-                                                    int *__restrict__ fast)
+                                                    const float *__restrict__ row1, int stride,
+                                                    int64_t np, int *__restrict__ fast)
 {
     __shared__ int turn[2];
     if (threadIdx.x < 2) turn[threadIdx.x] = FAST_MAX;
     __syncthreads();
-    const int n = (int)(np < FAST_MAX ? np : FAST_MAX);
+    const int n = (int)(np < FAST_MAX + 1 ? np : FAST_MAX + 1);
+    float v[2][FAST_MAX / 1024][2];
+    const float up[2] = {row0[stride] - row0[0], row1[stride] - row1[0]};
+#pragma unroll
+    for (int r = 0; r < 2; ++r)
+#pragma unroll
+        for (int t = 0; t < FAST_MAX / 1024; ++t) {
+            const int64_t p = (int64_t)min((int)threadIdx.x + t * 1024, n - 2) * stride;
+            v[r][t][0] = (r ? row1 : row0)[p];
+            v[r][t][1] = (r ? row1 : row0)[p + stride];
+        }
+#pragma unroll
     for (int r = 0; r < 2; ++r) {
-        const float *row = r ? row1 : row0;
-        const float up = row[1] - row[0];
         int first = FAST_MAX;
-        for (int p = threadIdx.x + 1; p + 1 < n; p += 1024)
-            if (first == FAST_MAX && (row[p + 1] - row[p]) * up < 0.0f) first = p + 1;
+#pragma unroll
+        for (int t = FAST_MAX / 1024 - 1; t >= 0; --t) {
+            const int p = min((int)threadIdx.x + t * 1024, n - 2);
+            if ((v[r][t][1] - v[r][t][0]) * up[r] < 0.0f) first = p + 1;
+        }
         if (first < FAST_MAX) atomicMin(&turn[r], first);
     }
     __syncthreads();
@@ -59,12 +72,10 @@ __global__ __launch_bounds__(1024) void k_fast_axis(const float *__restrict__ ro
     }
 }
 
-int launch_fast_axis(const float *ttx, int ntx, const float *trx, int nrx, int64_t np, int *fast,
+int launch_fast_axis(const float *row0, const float *row1, int stride, int64_t np, int *fast,
                      hipStream_t s)
 {
-    const float *t = nrx >= 2 ? trx : ttx;
-    const int64_t last = (nrx >= 2 ? nrx : ntx) - 1;
-    hipLaunchKernelGGL(k_fast_axis, dim3(1), dim3(1024), 0, s, t, t + last * np, np, fast);
+    hipLaunchKernelGGL(k_fast_axis, dim3(1), dim3(1024), 0, s, row0, row1, stride, np, fast);
     return check_launch("fast axis");
 }
 
@@ -76,7 +87,9 @@ int launch_das_wave(int gk, const DasArgs &a0, int max_part, float *partial, int
     // pixels of unknown order over tables: patches of the grid they form
     // (images of some tiles only; a small one fits the caches in any order)
     if (a.geo == 0 && !a.perm && fast && a.np >= 4096) {
-        if (int rc = launch_fast_axis(a.ttx, a.ntx, a.trx, a.nrx, a.np, fast, s)) return rc;
+        const float *row = a.nrx >= 2 ? a.trx : a.ttx;
+        const int64_t last = (a.nrx >= 2 ? a.nrx : a.ntx) - 1;
+        if (int rc = launch_fast_axis(row, row + last * a.np, 1, a.np, fast, s)) return rc;
         w.fast = fast;
     }
     w.nhalf = (float)a.nsrc - 0.5f;

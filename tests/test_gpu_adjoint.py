@@ -306,3 +306,23 @@ def test_das_beamformer_differentiates_synthetic_geometry_forward(mode, interp):
     lhs = float((out.detach().double() * G.double()).sum())
     rhs = float((rf.detach().double() * grf.double()).sum())
     assert abs(lhs - rhs) <= 1e-5 * (abs(lhs) + 1e-30), (lhs, rhs)
+
+
+@pytest.mark.parametrize("ntx,nrx,npx,nfr", [(1, 3, 1, 1), (2, 130, 64, 1), (130, 2, 65, 2), (5, 9, 255, 3),
+                                             (3, 17, 256, 1), (9, 8, 700, 1)])
+@pytest.mark.parametrize("kind", ["linear", "cubic", "korder_cubic"])
+def test_adjoint_at_tile_and_block_edges(kind, ntx, nrx, npx, nfr):
+    """Partial 64-pixel tiles, inner axes of more than one LDS block (the sums go
+    on from the stored gradients), images below and at the 256 pixels from
+    which the bins take the two-instruction conversion; weights of either sign
+    with some below the threshold.  Bar: 1e-4 of the FP64 gradient's peak, as
+    above."""
+    arrs = list(_case(41 + npx, ntx=ntx, nrx=nrx, np_=npx, nfr=nfr))
+    t0, dt = arrs[5:]
+    arrs = arrs[:5]
+    gout = np.random.default_rng(42).standard_normal((nfr, npx)).astype(np.float32)
+    out, g = _grads_gpu(arrs, t0, dt, kind, "tx_and_rx", 1e-2, gout)
+    ref_out, gr = _grads_ref(arrs, t0, dt, kind, "tx_and_rx", 1e-2, gout)
+    assert np.max(np.abs(out - ref_out)) <= 1e-4 * np.max(np.abs(ref_out))
+    for name, a, b in zip(NAMES, g, gr):
+        assert np.max(np.abs(a - b)) <= 1e-4 * np.max(np.abs(b)), name

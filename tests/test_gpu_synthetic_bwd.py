@@ -196,3 +196,23 @@ def test_headline_c0_gradient_matches_fp64_central_differences():
     print(f"  d energy / d c0: adjoint {float(gc):.6e}, FP64 central difference of the "
           f"linearised loss {fd:.6e}", flush=True)
     assert abs(float(gc) - fd) <= 1e-3 * abs(fd), (float(gc), fd)
+
+
+@pytest.mark.parametrize("thresh", [0.0, 0.5, 1.5])
+@pytest.mark.parametrize("kind", ["linear", "cubic"])
+def test_synthetic_adjoint_at_thresholds(kind, thresh):
+    """Zero weights that count (0), that do not (0.5: the delays go through the
+    geometry's delay table) and a threshold above every weight, against the
+    tables bit for bit; c0 alone equals c0 beside the other gradients."""
+    import torch
+    from pycbf_amd.gpu.autograd import das_synthetic
+    w = small_synthetic(seed=5, mode="div")
+    bf = _bf(w, {"kind": kind}, thresh=thresh)
+    rf = torch.as_tensor(w["rf"][None], device="cuda")
+    gout = torch.randn(bf._out_shape(1), generator=torch.Generator(device="cuda").manual_seed(3), device="cuda")
+    syn, tab = _grads(bf, rf, gout, True), _grads(bf, rf, gout, False)
+    for a, b in zip(syn, tab):
+        assert torch.equal(a, b) and (float(b.abs().max()) > 0) == (thresh < 1.0)
+    c0 = torch.tensor(float(bf.c0), dtype=torch.float32, requires_grad=True)
+    (g,) = torch.autograd.grad((das_synthetic(rf, bf, c0) * gout).sum(), [c0])
+    assert float(g) == float(syn[5])
