@@ -56,9 +56,20 @@ struct Stage {
 
 // ---------------------------------------------------------------------------
 // delay range per (tile, element) over the pixels that can contribute; a
-// workgroup takes one tile and TB_ELEMS elements (one barrier for all of them)
+// workgroup takes one tile and TB_ELEMS elements (one barrier for all of them).
+// The lowest bit of the upper bound says whether every pixel of the tile can
+// (the bound moves up by one ulp where its own bit says otherwise: a wider
+// range only widens a window).
 // ---------------------------------------------------------------------------
 constexpr int TB_ELEMS = 8;
+
+__device__ __forceinline__ float with_low_bit(float v, bool bit)
+{
+    const uint32_t u = __float_as_uint(v);
+    if ((u & 1u) == (bit ? 1u : 0u) || !(fabsf(v) < INFINITY)) return v;
+    if (v == 0.0f) return __uint_as_float(1u);
+    return __uint_as_float(v > 0.0f ? u + 1u : u - 1u);
+}
 
 template <int GEO>
 __global__ __launch_bounds__(256) void k_tile_bounds(DasArgs A)
@@ -75,10 +86,12 @@ __global__ __launch_bounds__(256) void k_tile_bounds(DasArgs A)
         for (int d = 0; d < GEO; ++d) pv[d] = A.pvec[p * GEO + d];
     }
     __shared__ float wl[TB_ELEMS][4], wh[TB_ELEMS][4];
+    __shared__ int wf[TB_ELEMS][4];
     const int w = threadIdx.x >> 6;
     for (int k = 0; k < TB_ELEMS && e0 + k < ne; ++k) {
         const int e = e0 + k;  // [0, ntx): tx element, [ntx, ntx+nrx): rx element
         float lo = INFINITY, hi = -INFINITY;
+        bool skipped = false;
         if (in) {
             const bool tx = e < A.ntx;
             float tau = 0.0f, apod = 0.0f;
@@ -87,7 +100,9 @@ __global__ __launch_bounds__(256) void k_tile_bounds(DasArgs A)
             const bool used =
                 (tau == tau) && (!(A.thresh > 0.0f) || (apod != 0.0f && apod == apod));
             if (used) lo = hi = tau;
+            skipped = !used;
         }
+        const int full = __any(skipped) ? 0 : 1;
 #pragma unroll
         for (int off = 32; off > 0; off >>= 1) {
             lo = fminf(lo, __shfl_xor(lo, off, 64));
@@ -96,6 +111,7 @@ __global__ __launch_bounds__(256) void k_tile_bounds(DasArgs A)
         if ((threadIdx.x & 63) == 0) {
             wl[k][w] = lo;
             wh[k][w] = hi;
+            wf[k][w] = full;
         }
     }
     __syncthreads();
@@ -105,7 +121,7 @@ __global__ __launch_bounds__(256) void k_tile_bounds(DasArgs A)
         const float hi = fmaxf(fmaxf(wh[k][0], wh[k][1]), fmaxf(wh[k][2], wh[k][3]));
         float *b = const_cast<float *>(A.bounds) + (tile * ne + e0 + k) * 2;
         b[0] = lo;
-        b[1] = hi;
+        b[1] = with_low_bit(hi, (wf[k][0] & wf[k][1] & wf[k][2] & wf[k][3]) != 0);
     }
 }
 
@@ -399,10 +415,10 @@ __global__ __launch_bounds__(LDS_BLOCK) void k_das_lds(DasArgs A)
 // aligned entry at or just below its first entry (rows are 8-byte aligned; the
 // parity of row * (nt + 1) + lo says which), and each frame owns CH chunk
 // slots, so chunk q of the staged block lands at byte 16 q.  Per outer
-// element one pass computes every inner channel's window into an LDS table;
-// channel b + 1 is in flight while b is evaluated (two LDS buffers, one
-// barrier per staged channel).  Nothing in the evaluation of channel b waits
-// on the DMA of channel b + 1: the buffers are separate LDS objects (a read
+// element one pass lists the inner channels with a window in LDS; the next
+// channel of the list is in flight while one is evaluated (two LDS buffers, one
+// barrier per channel).  Nothing in the evaluation of a channel waits on the
+// DMA of the next: the buffers are separate LDS objects (a read
 // of one is known not to alias the DMA into the other), geometry packs come
 // through the scalar cache and table entries are fetched a channel ahead.
 // Windows wider than the slot take direct global gathers, in a loop after
@@ -412,7 +428,7 @@ __global__ __launch_bounds__(LDS_BLOCK) void k_das_lds(DasArgs A)
 // quotient it rounds like the division (recip_division_exact): the same
 // delays and indices with three VALU instructions instead of a division.
 // ---------------------------------------------------------------------------
-constexpr int DMA_MAXB = 256;    // inner channels per outer element (window table)
+constexpr int DMA_MAXB = 256;    // inner channels per outer element (window list, one per thread)
 constexpr int DMA_CHUNKS = 768;  // 16-byte chunks per buffer (12 KB), all frames
 
 // one (y, h*y2) table entry as read from a staging buffer
@@ -424,8 +440,24 @@ typedef __attribute__((address_space(3))) void lds_void;
 typedef const __attribute__((address_space(1))) void glb_void;
 
 // FODD: a frame's rows span an odd number of table entries, so the rows of
-// consecutive frames start on alternating 8-byte parities
-template <int SUM, int FC, int GEO, bool OUTER_TX, bool FODD>
+// consecutive frames start on alternating 8-byte parities.
+// UNIT (geometry, thresh in (0, 1], t0 = 0, the last sample time on a knot of
+// the trace): a sample's weight is 1 or it does not count.  A pixel that does
+// not use an element holds a NaN delay, so no sample multiplies or tests a
+// weight; a receive element that every pixel of the tile uses (the low bit of
+// its delay range, FULL in the window table) skips the acceptance test; and
+// the time axis starts at zero.
+// The channels with a window are listed once per outer element, and the loop
+// walks the list with a channel's entry in scalar registers.  (Walking all
+// channels, four in ten of them with a window, and reading the window table
+// again for every test cost more in LDS latency and scalar instructions than
+// the unlisted evaluations themselves: 16 frames of 75 x 128 x 4096 onto 512 x
+// 512 5.56 ms; without the weights and the acceptance test, 2.70e9 -> 2.28e9
+// VALU instructions, 5.48 ms; with the list, 1.91e9 VALU and 0.72e9 scalar
+// ones (1.54e9), 4.43 ms.)  What bounds it now: VALU issue, 80 % of the cycles,
+// and the LDS reads of the stencil.
+
+template <int SUM, int FC, int GEO, bool OUTER_TX, bool FODD, bool UNIT>
 __global__ __launch_bounds__(LDS_BLOCK) void k_das_cubic_dma(DasArgs A)
 {
     constexpr int CH = DMA_CHUNKS / FC;     // chunk slots per frame row: 48 (FC 16) or 192
@@ -436,7 +468,9 @@ __global__ __launch_bounds__(LDS_BLOCK) void k_das_cubic_dma(DasArgs A)
     // that DMA's count
     __shared__ __align__(16) float lds0[DMA_CHUNKS * 4];
     __shared__ __align__(16) float lds1[DMA_CHUNKS * 4];
+    // channel | full << 8 | entries (staged ones) << 16, first entry
     __shared__ int2 wins[DMA_MAXB];
+    __shared__ int2 heads[LDS_BLOCK / 64];  // staged and wide channels of each wave's share
 
     uint32_t bx, by, bz;
     block_coords(A.xcd_remap, bx, by, bz);
@@ -513,6 +547,23 @@ __global__ __launch_bounds__(LDS_BLOCK) void k_das_cubic_dma(DasArgs A)
             elem_eval<GEO, true>(A, !OUTER_TX, b, p, pv, tau, apod);
         }
     };
+    // UNIT: the inner element's delay, NaN where the pixel does not use it
+    auto inner_delay = [&](int b, bool full) {
+        float tau, apod;
+        if (OUTER_TX && full) {
+            float pk[3];
+            load_pack(A.rxpack + (int64_t)b * PYCBF_RXPACK_FLOATS, pk);
+            float mag = 0.0f;
+#pragma unroll
+            for (int d = 0; d < GEO; ++d) {
+                const float di = pv[d] - pk[d];
+                mag += di * di;
+            }
+            return div_rn(sqrt_rn(mag), A.c0, A.rc0);
+        }
+        elem_eval<GEO, true>(A, !OUTER_TX, b, p, pv, tau, apod);
+        return apod != 0.0f ? tau : NAN;
+    };
 
     float acc[FC];
 #pragma unroll
@@ -521,45 +572,70 @@ __global__ __launch_bounds__(LDS_BLOCK) void k_das_cubic_dma(DasArgs A)
     for (int a = a0; a < a1; ++a) {
         float ta = 0.0f, wa = 0.0f;
         if (live) elem_eval<GEO, true>(A, OUTER_TX, a, p, pv, ta, wa);
+        if (UNIT && !(live && wa != 0.0f)) ta = NAN;
         const float amin = bnd[2 * (boff_a + a)], amax = bnd[2 * (boff_a + a) + 1];
-        for (int b = tid; b < nb; b += LDS_BLOCK) {
-            int lo, cnt;
-            channel_window<GK_CUBIC>(A, amin + bnd[2 * (boff_b + b)],
-                                     amax + bnd[2 * (boff_b + b) + 1], lo, cnt);
-            wins[b] = make_int2(lo, cnt);
+        // the inner channels with a window, in order: staged ones from the front of
+        // the list, those wider than a slot from its back (one channel per thread)
+        int lo = 0, cnt = 0;
+        bool full = false;
+        if (tid < nb) {
+            const float bmax = bnd[2 * (boff_b + tid) + 1];
+            channel_window<GK_CUBIC>(A, amin + bnd[2 * (boff_b + tid)], amax + bmax, lo, cnt);
+            full = UNIT && (__float_as_uint(bmax) & 1u);
+        }
+        const uint64_t ms = __ballot(cnt > 0 && cnt <= WINMAX), mw = __ballot(cnt > WINMAX);
+        if (lane == 0) heads[wave] = make_int2(__popcll(ms), __popcll(mw));
+        __syncthreads();
+        int ns = 0, nwide = 0, at = 0, atw = 0;
+#pragma unroll
+        for (int v = 0; v < LDS_BLOCK / 64; ++v) {
+            const int2 h = heads[v];
+            if (v < wave) {
+                at += h.x;
+                atw += h.y;
+            }
+            ns += h.x;
+            nwide += h.y;
+        }
+        ns = __builtin_amdgcn_readfirstlane(ns);
+        nwide = __builtin_amdgcn_readfirstlane(nwide);
+        const uint64_t below = (1ull << lane) - 1;
+        if (cnt > 0) {
+            const int k = cnt <= WINMAX ? at + __popcll(ms & below)
+                                        : DMA_MAXB - 1 - (atw + __popcll(mw & below));
+            wins[k] = make_int2(tid | (full ? 256 : 0) | (min(cnt, 0x7fff) << 16), lo);
         }
         __syncthreads();
 
+        // a channel of the list, the same in every lane: scalar registers, so its
+        // offsets are scalar arithmetic
+        struct Chan {
+            int b, lo, cnt, full;
+        };
+        auto chan = [&](int k) {
+            const int2 w = wins[k];
+            const int e = __builtin_amdgcn_readfirstlane(w.x);
+            return Chan{e & 255, __builtin_amdgcn_readfirstlane(w.y), e >> 16, e & 256};
+        };
         // table row of frame f (of this pass) for inner channel b
         auto row_of = [&](int b, int f) {
             const int tx = OUTER_TX ? a : b, rx = OUTER_TX ? b : a;
             return ((int64_t)(f0 + f) * nchan + (int64_t)tx * A.nrx + rx);
         };
-        auto staged = [&](int b) {
-            if (b >= nb) return false;
-            const int2 w = wins[b];
-            return w.y > 0 && w.y <= WINMAX;
-        };
-        // issue the DMA of channel b into buffer buf (workgroup-uniform condition)
-        auto dma = [&](int b, auto bufc) {
+        // issue the DMA of channel c into buffer buf (workgroup-uniform condition)
+        auto dma = [&](const Chan &c, auto bufc) {
             constexpr int buf = decltype(bufc)::value;
-            if (!staged(b)) return;
-            const int2 w = wins[b];
-            // the window is the same in every lane (one LDS word): scalar
-            // registers, so the channel's offset is scalar arithmetic
-            const int wx = __builtin_amdgcn_readfirstlane(w.x);
-            const int wy = __builtin_amdgcn_readfirstlane(w.y);
-            // entry wx of the channel's row, offset from the frame's table and
-            // its parity in frame 0 (workgroup-uniform)
-            const int64_t cho = row_of(b, -f0) * rowlen + wx;
+            // the window's first entry in the channel's row, offset from the
+            // frame's table, and its parity in frame 0 (workgroup-uniform)
+            const int64_t cho = row_of(c.b, -f0) * rowlen + c.lo;
             const int cpar = (int)(cho & 1);
 #pragma unroll
             for (int k = 0; k < NI; ++k) {
-                // the row's first staged entry is wx - par, 16-byte aligned
-                // (row r-1's last if -1); its nch = (wy + par + 1) / 2 chunks
+                // the row's first staged entry is lo - par, 16-byte aligned (row
+                // r-1's last if -1); its nch = (cnt + par + 1) / 2 chunks
                 const int par = FODD ? (dma_par[k] ^ cpar) : cpar;
-                const uint32_t c = (uint32_t)min(dma_c[k], (wy + par - 1) >> 1);
-                const float *src = dma_src[k] + (cho - par) * 2 + 4 * c;
+                const uint32_t q = (uint32_t)min(dma_c[k], (c.cnt + par - 1) >> 1);
+                const float *src = dma_src[k] + (cho - par) * 2 + 4 * q;
                 float *dst = (buf ? lds1 : lds0) + (k * (LDS_BLOCK / 64) + wave) * 64 * 4;
                 __builtin_amdgcn_global_load_lds((glb_void *)src, (lds_void *)dst, 16, 0, 0);
             }
@@ -572,34 +648,43 @@ __global__ __launch_bounds__(LDS_BLOCK) void k_das_cubic_dma(DasArgs A)
             wgt = OUTER_TX ? wa * wb : wb * wa;
             x = OUTER_TX ? ta + tb : tb + ta;
         };
-        // a staged channel (window of 1 .. WINMAX entries) from LDS buffer buf
-        auto compute = [&](int b, auto bufc, const float(&d)[NIN]) {
+        // a staged channel from LDS buffer buf
+        auto compute = [&](const Chan &c, auto bufc, const float(&d)[NIN]) {
             constexpr int buf = decltype(bufc)::value;
-            const int2 w = wins[b];
-            if (!(w.y > 0 && w.y <= WINMAX)) return;
-            float x, wgt;
-            delay(b, d, x, wgt);
+            float x, wgt = 1.0f, xlead, xlag;
             int j = 0;
-            if (!(live && fabsf(wgt) >= A.thresh &&
-                  knot_index_rn(x, A.t0, A.dt, A.rdt, A.tmax, A.nsrc, j)))
-                return;
-            const float xlead = A.t0 + A.dt * (float)(j + 1);
-            const float xlag = A.t0 + A.dt * (float)j;
+            if (UNIT) {
+                x = ta + inner_delay(c.b, c.full != 0);
+                if (!(x >= 0.0f && x <= A.tmax)) return;
+                const float jf = truncf(div_rn(x, A.dt, A.rdt));
+                j = (int)jf;
+                xlead = A.dt * (jf + 1.0f);
+                xlag = A.dt * jf;
+            } else {
+                delay(c.b, d, x, wgt);
+                if (!(live && fabsf(wgt) >= A.thresh &&
+                      knot_index_rn(x, A.t0, A.dt, A.rdt, A.tmax, A.nsrc, j)))
+                    return;
+                xlead = A.t0 + A.dt * (float)(j + 1);
+                xlag = A.t0 + A.dt * (float)j;
+            }
             float ka = (xlead - x) * A.rdt;
             float kb = (x - xlag) * A.rdt;
             float kc = __builtin_fmaf(ka * ka, ka, -ka);
             float kd = __builtin_fmaf(kb * kb, kb, -kb);
-            ka *= wgt;
-            kb *= wgt;
-            kc *= wgt;
-            kd *= wgt;
+            if (!UNIT) {
+                ka *= wgt;
+                kb *= wgt;
+                kc *= wgt;
+                kd *= wgt;
+            }
             // row parity of frame f: that of frame 0, flipped every frame when a
             // frame's rows span an odd number of entries
-            const int par0 = (int)((row_of(b, 0) * rowlen + w.x) & 1);
+            const int par0 = (int)((row_of(c.b, 0) * rowlen + c.lo) & 1);
             // every frame slot: those of frames past nf hold copies of frame
             // nf - 1 and feed sums that are never stored; straight-line code
             // lets the LDS reads of all frames overlap
-            const YZ *L = (const YZ *)(buf ? lds1 : lds0) + (j - w.x);
+            const YZ *L = (const YZ *)(buf ? lds1 : lds0) + (j - c.lo);
 #pragma unroll
             for (int g = 0; g < FC; g += FG) {
                 const YZ *Lg = L + (g / FG) * fg_step;
@@ -617,40 +702,48 @@ __global__ __launch_bounds__(LDS_BLOCK) void k_das_cubic_dma(DasArgs A)
             }
         };
 
-        bool wide = false;  // a channel's window exceeds the slot (workgroup-uniform)
-        // channel b: issue the DMA of channel b + 1 and the loads of its inner
-        // element's inputs (into dn, when some pixel of the tile takes a
-        // sample of it), evaluate channel b from LDS with inputs dc; the wait
-        // that ends the step covers both, so no wait inside a step holds its
-        // evaluation behind the next channel's DMA
-        auto step = [&](int b, auto bufc, const float(&dc)[NIN], float(&dn)[NIN]) {
-            constexpr int buf = decltype(bufc)::value;  // b & 1
-            dma(b + 1, std::integral_constant<int, buf ^ 1>());
-            if (b + 1 < nb && wins[b + 1].y > 0) inner_fetch(b + 1, dn);
-            wide |= wins[b].y > WINMAX;
-            compute(b, bufc, dc);
-            // this wave's DMA of channel b + 1 has landed; the barrier makes
-            // every wave's land, and frees buffer buf for channel b + 2
+        // channel k of the list: issue the DMA of channel k + 1 and the loads of
+        // its inner element's inputs (into dn), evaluate channel k from LDS with
+        // inputs dc; the wait that ends the step covers both, so no wait inside a
+        // step holds its evaluation behind the next channel's DMA
+        auto step = [&](int k, auto bufc, const Chan &c, Chan &nx, const float(&dc)[NIN],
+                        float(&dn)[NIN]) {
+            constexpr int buf = decltype(bufc)::value;  // k & 1
+            if (k + 1 < ns) {
+                nx = chan(k + 1);
+                dma(nx, std::integral_constant<int, buf ^ 1>());
+                inner_fetch(nx.b, dn);
+            }
+            compute(c, bufc, dc);
+            // this wave's DMA of channel k + 1 has landed; the barrier makes every
+            // wave's land, and frees buffer buf for channel k + 2
             __builtin_amdgcn_s_waitcnt(0);
-            if (staged(b) || staged(b + 1)) __syncthreads();
+            __syncthreads();
         };
         float d0[NIN], d1[NIN];
-        if (wins[0].y > 0) inner_fetch(0, d0);
-        dma(0, std::integral_constant<int, 0>());
-        __builtin_amdgcn_s_waitcnt(0);
-        if (staged(0)) __syncthreads();
-        for (int b = 0; b < nb; b += 2) {
-            step(b, std::integral_constant<int, 0>(), d0, d1);
-            if (b + 1 < nb) step(b + 1, std::integral_constant<int, 1>(), d1, d0);
+        if (ns > 0) {
+            Chan c0 = chan(0), c1 = c0;
+            inner_fetch(c0.b, d0);
+            dma(c0, std::integral_constant<int, 0>());
+            __builtin_amdgcn_s_waitcnt(0);
+            __syncthreads();
+            for (int k = 0; k < ns; k += 2) {
+                step(k, std::integral_constant<int, 0>(), c0, c1, d0, d1);
+                if (k + 1 < ns) step(k + 1, std::integral_constant<int, 1>(), c1, c0, d1, d0);
+            }
         }
         // channels whose window exceeds a staging slot: direct gathers, after
         // the staged ones (a loop of its own keeps the staged loop's registers)
-        for (int b = 0; wide && b < nb; ++b) {
-            if (wins[b].y <= WINMAX) continue;
-            float x, wgt;
-            inner_fetch(b, d0);
-            delay(b, d0, x, wgt);
-            if (!(live && fabsf(wgt) >= A.thresh)) continue;
+        for (int k = 0; k < nwide; ++k) {
+            const int b = chan(DMA_MAXB - 1 - k).b;
+            float x, wgt = 1.0f;
+            if (UNIT) {
+                x = ta + inner_delay(b, false);
+            } else {
+                inner_fetch(b, d0);
+                delay(b, d0, x, wgt);
+                if (!(live && fabsf(wgt) >= A.thresh)) continue;
+            }
             const int tx = OUTER_TX ? a : b, rx = OUTER_TX ? b : a;
             float v[FC];
             bool ok = false;
@@ -679,15 +772,30 @@ __global__ __launch_bounds__(LDS_BLOCK) void k_das_cubic_dma(DasArgs A)
     }
 }
 
+template <int SUM, int FC, bool OT, bool FODD, int GEO>
+static void cubic_dma_unit(const DasArgs &a, dim3 grid, hipStream_t s)
+{
+    // see UNIT at the kernel
+    const bool unit = a.thresh > 0.0f && a.thresh <= 1.0f && a.t0 == 0.0f &&
+                      (int)(a.tmax / a.dt) <= a.nsrc - 1;
+    if (unit)
+        hipLaunchKernelGGL((k_das_cubic_dma<SUM, FC, GEO, OT, FODD, true>), grid, dim3(LDS_BLOCK),
+                           0, s, a);
+    else
+        hipLaunchKernelGGL((k_das_cubic_dma<SUM, FC, GEO, OT, FODD, false>), grid, dim3(LDS_BLOCK),
+                           0, s, a);
+}
+
 template <int SUM, int FC, bool OT, bool FODD>
 static void cubic_dma_launch(int geo, const DasArgs &a, dim3 grid, hipStream_t s)
 {
     if (geo == 3)
-        hipLaunchKernelGGL((k_das_cubic_dma<SUM, FC, 3, OT, FODD>), grid, dim3(LDS_BLOCK), 0, s, a);
+        cubic_dma_unit<SUM, FC, OT, FODD, 3>(a, grid, s);
     else if (geo == 2)
-        hipLaunchKernelGGL((k_das_cubic_dma<SUM, FC, 2, OT, FODD>), grid, dim3(LDS_BLOCK), 0, s, a);
+        cubic_dma_unit<SUM, FC, OT, FODD, 2>(a, grid, s);
     else
-        hipLaunchKernelGGL((k_das_cubic_dma<SUM, FC, 0, OT, FODD>), grid, dim3(LDS_BLOCK), 0, s, a);
+        hipLaunchKernelGGL((k_das_cubic_dma<SUM, FC, 0, OT, FODD, false>), grid, dim3(LDS_BLOCK),
+                           0, s, a);
 }
 
 template <int SUM, int FC, bool OT>
