@@ -44,7 +44,7 @@ int launch_spline_coefs(const float *rf, int64_t nch, int32_t nt, float dt, floa
                         float2 *coef, hipStream_t s);
 int launch_spline_y2(const float *rf, int64_t nch, int32_t nt, float dt, float *uscr, float *y2,
                      hipStream_t s);
-// Samples per lane (32 or 64) of the one-wave-per-channel spline sweeps for
+// Samples per lane (32 or 64) of the one-wave-per-channel spline adjoint for
 // traces of nt samples, or 0 for the one-lane-per-channel sweeps (nt > 4096,
 // or PYCBF_SPLINE_SEG=0 in the environment at the call).
 int spline_seg_len(int32_t nt);

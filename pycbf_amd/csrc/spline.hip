@@ -1,8 +1,8 @@
 // Per-channel prefilters: turn each RF channel into a table the DAS gather
 // reads with one load per sample.
 //
-//  * k_spline_seg (nt <= 4096): natural cubic spline (tie_knots1D_fixed,
-//    pycbf/cpu/pycbf.c:114-166), one wave per channel, each lane sweeping a
+//  * k_spline_seg (nt <= 32768): natural cubic spline (tie_knots1D_fixed,
+//    pycbf/cpu/pycbf.c:114-166), one to eight waves per channel, each lane sweeping a
 //    segment from a verified carry; bit-identical second derivatives.
 //  * k_spline (longer channels): the same spline, one wave owns 64 channels;
 //    32-sample tiles are staged through LDS so that global loads/stores stay
@@ -224,9 +224,9 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3))) void k_
     }
 }
 
-// ---- segment-parallel sweeps: one wave per channel -------------------------
+// ---- segment-parallel sweeps -----------------------------------------------
 //
-// For nt <= 64*SEG, lane l of the wave owns the SEG consecutive samples
+// For nt <= 64*NW*SEG, lane l of a channel's waves owns the SEG consecutive samples
 // i0 = l*SEG .. i0+SEG-1 of one channel, held in registers.  Both sweeps of
 // tie_knots1D_fixed are first-order recurrences that contract by
 // |0.5/p| ~ 0.27 per step (p -> 1 + sqrt(3)/2), so a lane can start each
@@ -238,7 +238,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3))) void k_
 // After each sweep every guess is compared bit for bit with the value the
 // neighbouring lane computed.  A lane whose guess differs takes its
 // neighbour's value and recomputes its segment, until every carry agrees.
-// Lane 0's forward carry and lane 63's backward carry are the exact boundary
+// Lane 0's forward carry and the last lane's backward carry are the exact boundary
 // values, and a segment computed from an exact carry is exact, so agreement
 // of all carries means every segment equals the sequential sweep bit for bit,
 // whatever the data.  A guess misses only when the data's magnitude falls by
@@ -297,13 +297,40 @@ __device__ __forceinline__ bool bits_differ(float a, float b)
     return __float_as_uint(a) != __float_as_uint(b);
 }
 
-template <int MODE, int SEG>  // MODE 0: (y, dx^2/6*y2) gather table, 1: y2
-__global__ __launch_bounds__(64) void k_spline_seg(const float *__restrict__ rf, int nt, float dx,
-                                                   void *__restrict__ outp)
+// NW waves share a channel of up to 64 NW SEG samples (one for 4096; traces of
+// up to 32768 samples take two to eight): `lane` counts the workgroup's lanes, and
+// neighbours beyond a wave's edge are reached through LDS.  k_spline, one lane
+// per channel, waits on its serial chain whatever the channel count: 2106
+// channels of 4596 samples 1175 us, here 71; 1000 of 20 000 samples 5.2 ms, here
+// 0.13.  Two waves of 32-sample lanes for 2049 .. 4096 samples measured the same
+// as one of 64 (9600 channels 134 us; the 16-frame batch 2 % slower).
+template <int MODE, int SEG, int NW>  // MODE 0: (y, dx^2/6*y2) gather table, 1: y2
+__global__ __launch_bounds__(64 * NW) void k_spline_seg(const float *__restrict__ rf, int nt,
+                                                        float dx, void *__restrict__ outp)
 {
     static_assert(SEG % 32 == 0 && SEG >= SEG_WARM, "segments are whole 32-sample tiles");
-    __shared__ __align__(16) SplRow S[64];
+    constexpr int LANES = 64 * NW;
+    __shared__ __align__(16) SplRow S[LANES];
+    __shared__ float edge[NW > 1 ? LANES : 1];
     const int lane = threadIdx.x;
+    SplRow *Sw = S + (lane & ~63);  // this wave's rows of the tile
+    const int row0 = lane & ~63;
+    // the value of the lane before / after this one (its own at the ends)
+    auto from_left = [&](float v) {
+        if (NW == 1) return __shfl_up(v, 1);
+        __syncthreads();
+        edge[lane] = v;
+        __syncthreads();
+        return edge[lane > 0 ? lane - 1 : 0];
+    };
+    auto from_right = [&](float v) {
+        if (NW == 1) return __shfl_down(v, 1);
+        __syncthreads();
+        edge[lane] = v;
+        __syncthreads();
+        return edge[lane < LANES - 1 ? lane + 1 : lane];
+    };
+    auto any_lane = [&](bool b) { return NW == 1 ? __ballot(b) != 0 : __syncthreads_or(b) != 0; };
     const bool lane0 = lane == 0;
     const int64_t ch = blockIdx.x;
     const float *yrow = rf + ch * (int64_t)nt;
@@ -337,7 +364,7 @@ __global__ __launch_bounds__(64) void k_spline_seg(const float *__restrict__ rf,
             TileRegs r;
 #pragma unroll
             for (int q = 0; q < 8; ++q) {
-                const int k = (8 * q + (lane >> 3)) * SEG + 32 * t + c;
+                const int k = (row0 + 8 * q + ((lane & 63) >> 3)) * SEG + 32 * t + c;
                 F4u w{{0.0f, 0.0f, 0.0f, 0.0f}};
                 if (k + 4 <= nt) {
                     w = *reinterpret_cast<const F4u *>(yrow + k);
@@ -349,7 +376,7 @@ __global__ __launch_bounds__(64) void k_spline_seg(const float *__restrict__ rf,
                 r.q[q] = w;
             }
             if (t > 0) __syncthreads();  // previous tile read out
-            tile_to_lds(r, S);
+            tile_to_lds(r, Sw);
             __syncthreads();
             float part[32];
             row_read(S, part);
@@ -357,8 +384,8 @@ __global__ __launch_bounds__(64) void k_spline_seg(const float *__restrict__ rf,
             for (int e = 0; e < 32; ++e) y[32 * t + e] = part[e];
         }
     }
-    const float yl = __shfl_up(y[SEG - 1], 1);  // y_{i0-1}
-    const float yr = __shfl_down(y[0], 1);      // y_{i0+SEG}
+    const float yl = from_left(y[SEG - 1]);  // y_{i0-1}
+    const float yr = from_right(y[0]);       // y_{i0+SEG}
 
     // ---- forward sweep -----------------------------------------------------
     // guess of u_{i0-1}: u = 0 at i0-32, then i = i0-31 .. i0-1 over the left
@@ -393,9 +420,9 @@ __global__ __launch_bounds__(64) void k_spline_seg(const float *__restrict__ rf,
     float last = seg_forward<SEG>(y, yl, yr, dx, carry, i0, nt, p_inf, plo, lane0, v);
     // lanes with i0 > nt-2 hold no u values; their carries need not agree
     for (;;) {
-        const float want = __shfl_up(last, 1);
+        const float want = from_left(last);
         const bool redo = lane > 0 && i0 <= nt - 2 && bits_differ(carry, want);
-        if (__ballot(redo) == 0) break;
+        if (!any_lane(redo)) break;
         if (redo) {
             carry = want;
             last = seg_forward<SEG>(y, yl, yr, dx, carry, i0, nt, p_inf, plo, lane0, v);
@@ -409,8 +436,8 @@ __global__ __launch_bounds__(64) void k_spline_seg(const float *__restrict__ rf,
     for (int e = 0; e < 32; e += 4)  // u_{i0 .. i0+31}
         *reinterpret_cast<float4 *>(&S[lane][e]) = make_float4(v[e], v[e + 1], v[e + 2], v[e + 3]);
     __syncthreads();
-    float bcarry = 0.0f;  // lane 63: y2 beyond the channel is 0
-    if (lane < 63) {
+    float bcarry = 0.0f;  // last lane: y2 beyond the channel is 0
+    if (lane < LANES - 1) {
         float nxt = 0.0f;
 #pragma unroll
         for (int e = 28; e >= 0; e -= 4) {
@@ -424,9 +451,9 @@ __global__ __launch_bounds__(64) void k_spline_seg(const float *__restrict__ rf,
     }
     float first = seg_backward<SEG>(v, bcarry, y2f_inf, flo, lane0);
     for (;;) {
-        const float want = __shfl_down(first, 1);
-        const bool redo = lane < 63 && i0 < nt && bits_differ(bcarry, want);
-        if (__ballot(redo) == 0) break;
+        const float want = from_right(first);
+        const bool redo = lane < LANES - 1 && i0 < nt && bits_differ(bcarry, want);
+        if (!any_lane(redo)) break;
         if (redo) {
             // rebuild u from the exact forward carry, then substitute again
             bcarry = want;
@@ -452,7 +479,7 @@ __global__ __launch_bounds__(64) void k_spline_seg(const float *__restrict__ rf,
             __syncthreads();
 #pragma unroll
             for (int q = 0; q < 8; ++q) {
-                const int r = 8 * q + (lane >> 3);
+                const int r = row0 + 8 * q + ((lane & 63) >> 3);
                 const int f = 2 * (r * SEG + 16 * hh) + c;  // float index in the row
                 const float4 w = *reinterpret_cast<const float4 *>(&S[r][c]);
                 if (f + 4 <= 2 * nt) {
@@ -483,7 +510,7 @@ __global__ __launch_bounds__(64) void k_spline_seg(const float *__restrict__ rf,
             __syncthreads();
 #pragma unroll
             for (int q = 0; q < 8; ++q) {
-                const int r = 8 * q + (lane >> 3);
+                const int r = row0 + 8 * q + ((lane & 63) >> 3);
                 const int k = r * SEG + 32 * t + c;
                 const float4 w = *reinterpret_cast<const float4 *>(&S[r][c]);
                 if (k + 4 <= nt) {
@@ -500,10 +527,15 @@ __global__ __launch_bounds__(64) void k_spline_seg(const float *__restrict__ rf,
     }
 }
 
+static bool spline_segments()
+{
+    const char *e = getenv("PYCBF_SPLINE_SEG");
+    return !(e && atoi(e) == 0);
+}
+
 int spline_seg_len(int32_t nt)
 {
-    if (const char *e = getenv("PYCBF_SPLINE_SEG"))
-        if (atoi(e) == 0) return 0;
+    if (!spline_segments()) return 0;
     if (nt <= 64 * 32) return 32;
     if (nt <= 64 * 64) return 64;
     return 0;
@@ -515,19 +547,23 @@ static int launch_spline(const float *rf, int64_t nch, int32_t nt, float dt, flo
 {
     if (nch <= 0 || nt <= 0) return 0;
     if (nt > SPL_MAX_NT) return fail(1, "spline: nt %d exceeds %d samples", nt, SPL_MAX_NT);
-    switch (spline_seg_len(nt)) {
-    case 32:
-        hipLaunchKernelGGL((k_spline_seg<MODE, 32>), dim3((unsigned)nch), dim3(64), 0, s, rf,
-                           (int)nt, dt, out);
-        break;
-    case 64:
-        hipLaunchKernelGGL((k_spline_seg<MODE, 64>), dim3((unsigned)nch), dim3(64), 0, s, rf,
-                           (int)nt, dt, out);
-        break;
-    default:
+    const dim3 grid((unsigned)nch);
+    if (!spline_segments())
         hipLaunchKernelGGL(k_spline<MODE>, dim3((unsigned)((nch + 63) / 64)), dim3(64), 0, s, rf,
                            nch, (int)nt, dt, uscr, out);
-    }
+    else if (nt <= 64 * 32)
+        hipLaunchKernelGGL((k_spline_seg<MODE, 32, 1>), grid, dim3(64), 0, s, rf, (int)nt, dt, out);
+    else if (nt <= 64 * 64)
+        hipLaunchKernelGGL((k_spline_seg<MODE, 64, 1>), grid, dim3(64), 0, s, rf, (int)nt, dt, out);
+    else if (nt <= 2 * 64 * 64)
+        hipLaunchKernelGGL((k_spline_seg<MODE, 64, 2>), grid, dim3(128), 0, s, rf, (int)nt, dt, out);
+    else if (nt <= 4 * 64 * 64)
+        hipLaunchKernelGGL((k_spline_seg<MODE, 64, 4>), grid, dim3(256), 0, s, rf, (int)nt, dt, out);
+    else if (nt <= 8 * 64 * 64)
+        hipLaunchKernelGGL((k_spline_seg<MODE, 64, 8>), grid, dim3(512), 0, s, rf, (int)nt, dt, out);
+    else
+        hipLaunchKernelGGL(k_spline<MODE>, dim3((unsigned)((nch + 63) / 64)), dim3(64), 0, s, rf,
+                           nch, (int)nt, dt, uscr, out);
     return check_launch(MODE == 0 ? "spline coefficients" : "spline y2");
 }
 

@@ -67,9 +67,10 @@ __device__ __forceinline__ void tile_fetch(const float *base, int ld, int nrow, 
     }
 }
 
+// S: the wave's 64 rows
 __device__ __forceinline__ void tile_to_lds(const TileRegs &t, SplRow *S)
 {
-    const int lane = threadIdx.x;
+    const int lane = threadIdx.x & 63;
     const int c = 4 * (lane & 7);
 #pragma unroll
     for (int q = 0; q < 8; ++q)

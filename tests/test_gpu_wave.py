@@ -109,3 +109,33 @@ def test_wave_gather_over_grids_in_their_own_order(nx, nz, xfast):
     for kind in ("cubic", "linear"):
         got = das_tabbed(d(rf), *(d(t) for t in tabs), 0.0, DT, kind, "tx_and_rx", 1e-2).cpu().numpy()
         assert_close_to_peak(got, oracle.das_tabbed(rf, 0.0, DT, *tabs, kind=kind), 1e-5, kind)
+
+
+@pytest.mark.parametrize("data", ["normal", "bursts"])
+@pytest.mark.parametrize("nt", [4097, 8191, 8192, 8193, 16385, 32768, 32769])
+def test_spline_prefilter_over_several_waves_bitwise(nt, data):
+    """Channels shared by two to eight waves (and one sample past the longest),
+    dense data and bursts between zero runs of up to 200 samples (guessed
+    carries that have to be recomputed across a wave's edge): second
+    derivatives bit for bit the reference recurrence's."""
+    import torch
+    from pycbf_amd.gpu import _engine as E
+    rng = np.random.default_rng(nt)
+    nch, dt = 5, np.float32(2.5e-8)
+    rf = rng.standard_normal((nch, nt)).astype(np.float32)
+    if data == "bursts":
+        on = np.zeros((nch, nt), bool)
+        for c in range(nch):
+            k = 0
+            while k < nt:
+                n = int(rng.integers(1, 8))
+                on[c, k:k + n] = True
+                k += n + int(rng.integers(1, 200))
+        rf *= on
+    x = torch.as_tensor(rf, device="cuda")
+    wsb = E.lib.pycbf_spline_workspace_bytes(nch, nt)
+    ws = torch.empty(wsb, dtype=torch.uint8, device="cuda")
+    y2 = torch.empty((nch, nt), dtype=torch.float32, device="cuda")
+    E.check(E.lib.pycbf_spline_y2(E.ptr(x), nch, nt, float(dt), E.ptr(y2), E.ptr(ws), wsb, E.stream_of(x.device)), "y2")
+    ref = np.stack([oracle.spline_y2(r, dt) for r in rf])
+    assert np.array_equal(y2.cpu().numpy().view(np.uint32), ref.view(np.uint32))
