@@ -126,3 +126,31 @@ def test_demod_full_image_timing():
     ms = (time.perf_counter() - t0) * 1e2
     print(f"demod 512 x 4096 -> {tuple(iq.shape)}: {ms:.3f} ms per call", flush=True)
     assert bool(torch.isfinite(torch.view_as_real(iq)).all())
+
+
+@pytest.mark.parametrize("n", [512, 1024, 2048, 4096])
+@pytest.mark.parametrize("m", [64, 65, 128, 129, 256, 257, 511, 512, 513, 1000])
+def test_demod_fft_sizes(n, m):
+    """Every pair of transform sizes on both sides of the register kernel's
+    limit (256 points), bands that fill the convolution to its last point,
+    one that begins at bin 0 and one that ends at n / 2, fewer lines than
+    workgroups and more; float32 input rounding plus float32 accumulation
+    over the log2 n stages, as above."""
+    import torch
+    from pycbf_amd.gpu.demod import fft_tables, fft_tukey_demod
+    if m > n // 2 + 1:
+        pytest.skip("more bins than the axis has")
+    print(f"demod fft n={n} bins={m}", flush=True)
+    rng = np.random.default_rng(n + m)
+    for lo, rows in ((0, 3), (n // 2 + 1 - m, 5), ((n // 2 + 1 - m) // 2, 9001)):
+        kmin, kmax = lo / n, (lo + m - 1) / n
+        assert od.band(n, kmin, kmax, 1.0) == (lo, lo + m)
+        if fft_tables(n, kmin, kmax, 1.0) is None:
+            continue
+        x = rng.standard_normal((rows, n)).astype(np.float32)
+        got = fft_tukey_demod(torch.as_tensor(x, device="cuda"), kmin, kmax, 1.0, method="fft")
+        g = got.cpu().numpy()
+        pick = np.unique(np.r_[0:min(rows, 64), max(0, rows - 64):rows])
+        want = od.fft_tukey_demod(x[pick].astype(np.float64), kmin, kmax, 1.0)
+        assert g.shape == (rows,) + want.shape[1:] and np.isfinite(g).all()
+        assert np.abs(g[pick] - want).max() <= 2e-5 * np.abs(want).max()
