@@ -231,8 +231,8 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3))) void k_
 // tie_knots1D_fixed are first-order recurrences that contract by
 // |0.5/p| ~ 0.27 per step (p -> 1 + sqrt(3)/2), so a lane can start each
 // sweep from a guessed carry a little outside its segment:
-//  * forward: u = 0 at i0-32, run over the left neighbour's last 31 samples
-//    to get a guess of u_{i0-1};
+//  * forward: u = 0 at i0-32, run over the left neighbour's last 31 right-hand
+//    sides to get a guess of u_{i0-1};
 //  * backward: y2 = 0 at i0+SEG+32, run over the right neighbour's first 32
 //    u values to get a guess of y2_{i0+SEG}.
 // After each sweep every guess is compared bit for bit with the value the
@@ -247,8 +247,8 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3))) void k_
 //
 // Global memory is touched once per sample: the channel is read in coalesced
 // 64 x 32 tiles (row l = 32 samples of lane l's segment) and transposed
-// through one LDS tile; the output goes back the same way.  Compared with
-// k_spline there is no scratch round trip and no second read of the channel.
+// through one LDS tile; the table goes back by whole segments, the second
+// derivatives by tiles.  Compared with k_spline there is no scratch round trip and no second read of the channel.
 constexpr int SEG_WARM = 32;  // warm-up length of both sweeps (samples)
 
 // Fills u_{i0+c} (c < SEG) from the exact or guessed carry u = u_{i0-1}.
@@ -260,11 +260,17 @@ __device__ __forceinline__ float seg_forward(const float (&y)[SEG], float yl, fl
                                              float u, int i0, int nt, float p_inf,
                                              const float (&plo)[9], bool lane0, float (&v)[SEG])
 {
-    float d_prev = (y[0] - yl) / dx;
+    // opaque copies: this sweep runs for few lanes, and what it shares with the
+    // fast one is not to be held in registers for it
+    float yc = y[0];
+    asm volatile("" : "+v"(yc));
+    float d_prev = (yc - yl) / dx;
 #pragma unroll
     for (int c = 0; c < SEG; ++c) {
-        const float ynext = (c + 1 < SEG) ? y[c + 1] : yr;
-        const float d = (ynext - y[c]) / dx;
+        float ynext = (c + 1 < SEG) ? y[c + 1] : yr;
+        asm volatile("" : "+v"(ynext));
+        const float d = (ynext - yc) / dx;
+        yc = ynext;
         const float g = 6.0f * (d - d_prev) / (2.0f * dx);
         d_prev = d;
         // p_i = 0.5*y2f[i-1] + 2 differs from p_inf only for i < 9 (lane 0)
@@ -276,6 +282,33 @@ __device__ __forceinline__ float seg_forward(const float (&y)[SEG], float yl, fl
     }
     return u;
 }
+
+// x / d from r = 1 / d rounded to nearest, rounded as the division is: two
+// corrections by the exact remainder (P. Markstein, "Computation of elementary
+// functions on the IBM RISC System/6000 processor", 1990: the second starts
+// within one unit in the last place).  Exact remainders need x = +-0 or |x| a
+// factor 2^48 above the smallest float, and |x / d| normal.  Five operations
+// against eleven, one of them a quarter-rate reciprocal.
+__device__ __forceinline__ float div_rn(float x, float d, float r)
+{
+    const float q0 = x * r;
+    const float q1 = __builtin_fmaf(-__builtin_fmaf(q0, d, -x), r, q0);
+    return __builtin_fmaf(-__builtin_fmaf(q1, d, -x), r, q1);
+}
+
+// |v| - 1 in units of the last place: 0 is the largest unsigned and the
+// smallest signed value, NaN a large one of both
+__device__ __forceinline__ uint32_t mag_bits(float v)
+{
+    return (__float_as_uint(v) & 0x7fffffffu) - 1u;
+}
+
+// The inputs that keep every division of the fast sweep in div_rn's range: dx
+// in [2^-40, 1], samples 0 or 2^-46 <= |y| <= 2^40 (so that differences and
+// difference quotients are 0 or >= 2^-93 and g <= 2^124), and u values 0 or
+// >= 2^-96 (they decay through stretches of zeros).
+constexpr uint32_t FAST_YLO = (127u - 46u) << 23, FAST_YHI = (127u + 40u) << 23;
+constexpr uint32_t FAST_ULO = (127u - 96u) << 23;
 
 // y2_{i0+c} = y2f[i0+c] * y2_{i0+c+1} + u_{i0+c}, c = SEG-1 .. 0, in place,
 // from the carry y2_{i0+SEG}.  Returns y2_{i0}.
@@ -292,6 +325,14 @@ __device__ __forceinline__ float seg_backward(float (&v)[SEG], float nxt, float 
     return nxt;
 }
 
+// the wave's own tile rows change hands between its lanes
+__device__ __forceinline__ void tile_sync()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 __device__ __forceinline__ bool bits_differ(float a, float b)
 {
     return __float_as_uint(a) != __float_as_uint(b);
@@ -299,11 +340,22 @@ __device__ __forceinline__ bool bits_differ(float a, float b)
 
 // NW waves share a channel of up to 64 NW SEG samples (one for 4096; traces of
 // up to 32768 samples take two to eight): `lane` counts the workgroup's lanes, and
-// neighbours beyond a wave's edge are reached through LDS.  k_spline, one lane
-// per channel, waits on its serial chain whatever the channel count: 2106
-// channels of 4596 samples 1175 us, here 71; 1000 of 20 000 samples 5.2 ms, here
-// 0.13.  Two waves of 32-sample lanes for 2049 .. 4096 samples measured the same
-// as one of 64 (9600 channels 134 us; the 16-frame batch 2 % slower).
+// neighbours beyond a wave's edge are reached through LDS.
+//
+// What bounds it: the channel's 4 bytes read and 8 written per sample.  With
+// the three divisions per sample as the compiler expands them it was VALU work
+// (85 instructions per sample, 51 of them in the divisions and the warm-up),
+// and with 128-byte pieces of every segment per output pass the unaligned rows
+// of the table were written as halves of lines, which L2 no longer joined
+// once the arithmetic was out of the way (9600 x 4096: 134 us before, 147
+// with the cheap divisions alone, 99 with whole-segment passes as well: 4.8
+// TB/s; 153 600 x 4096 1735 -> 1370, 5.5 TB/s; 9600 x 2048 67 -> 43;
+// 3968 x 5000 120 -> 83).  Reading by whole segments as well put each pass's
+// loads behind the last one's: 135 at 9600 x 4096.  Two waves of 32-sample
+// lanes for 2049 .. 4096 samples measured the same on one frame and 1 % slower
+// on sixteen.  k_spline, one lane per channel, waits on its serial chain
+// whatever the channel count: 2106 channels of 4596 samples 1175 us, here 56;
+// 1000 of 20 000 samples 5.2 ms, here 0.10.
 template <int MODE, int SEG, int NW>  // MODE 0: (y, dx^2/6*y2) gather table, 1: y2
 __global__ __launch_bounds__(64 * NW) void k_spline_seg(const float *__restrict__ rf, int nt,
                                                         float dx, void *__restrict__ outp)
@@ -388,43 +440,80 @@ __global__ __launch_bounds__(64 * NW) void k_spline_seg(const float *__restrict_
     const float yr = from_right(y[0]);       // y_{i0+SEG}
 
     // ---- forward sweep -----------------------------------------------------
+    // the fast form first, in place: g, then u from it; bad = a division left
+    // the range of div_rn, the lane sweeps again with the divisions themselves
+    float v[SEG];
+    bool bad;
+    const float rdx = 1.0f / dx, dx2 = 2.0f * dx, rdx2 = 1.0f / dx2;
+    {
+        uint32_t mn = mag_bits(yl) < mag_bits(yr) ? mag_bits(yl) : mag_bits(yr);
+        int32_t mx = (int32_t)mag_bits(yl) > (int32_t)mag_bits(yr) ? (int32_t)mag_bits(yl)
+                                                                   : (int32_t)mag_bits(yr);
+        float d_prev = div_rn(y[0] - yl, dx, rdx);
+#pragma unroll
+        for (int c = 0; c < SEG; ++c) {
+            const uint32_t b = mag_bits(y[c]);
+            mn = b < mn ? b : mn;
+            mx = (int32_t)b > mx ? (int32_t)b : mx;
+            const float d = div_rn(((c + 1 < SEG) ? y[c + 1] : yr) - y[c], dx, rdx);
+            v[c] = div_rn(6.0f * (d - d_prev), dx2, rdx2);
+            d_prev = d;
+        }
+        bad = mn < FAST_YLO - 1u || mx > (int32_t)FAST_YHI || !(dx >= 0x1p-40f && dx <= 1.0f);
+    }
     // guess of u_{i0-1}: u = 0 at i0-32, then i = i0-31 .. i0-1 over the left
-    // neighbour's last 32 samples (still in the LDS tile)
+    // neighbour's last g values
+    __syncthreads();  // the samples are read out of the tile
+#pragma unroll
+    for (int e = 0; e < 32; e += 4)
+        *reinterpret_cast<float4 *>(&S[lane][e]) =
+            make_float4(v[SEG - 32 + e], v[SEG - 31 + e], v[SEG - 30 + e], v[SEG - 29 + e]);
+    __syncthreads();
+    const float rp_inf = 1.0f / p_inf;
     float carry = 0.0f;
     if (lane > 0) {
-        float w[32];
+        // only lane 1 of a 32-sample segment reaches i < 9 here
+        const bool low = (SEG == 32) && lane == 1;
+        float u = 0.0f;
 #pragma unroll
         for (int e = 0; e < 32; e += 4) {
             const float4 q4 = *reinterpret_cast<const float4 *>(&S[lane - 1][e]);
-            w[e] = q4.x;
-            w[e + 1] = q4.y;
-            w[e + 2] = q4.z;
-            w[e + 3] = q4.w;
-        }
-        // only lane 1 of a 32-sample segment reaches i < 9 here
-        const bool low = (SEG == 32) && lane == 1;
-        float d_prev = (w[1] - w[0]) / dx;
-        float u = 0.0f;
+            const float w[4] = {q4.x, q4.y, q4.z, q4.w};
 #pragma unroll
-        for (int c = 1; c < 32; ++c) {
-            const float ynext = (c + 1 < 32) ? w[c + 1] : y[0];
-            const float d = (ynext - w[c]) / dx;
-            const float g = 6.0f * (d - d_prev) / (2.0f * dx);
-            d_prev = d;
-            const float p = (c < 9 && low) ? plo[c < 9 ? c : 0] : p_inf;
-            u = (g - 0.5f * u) / p;
+            for (int c = e == 0 ? 1 : 0; c < 4; ++c) {
+                const bool lo = e + c < 9 && low;
+                const float p = lo ? plo[e + c < 9 ? e + c : 0] : p_inf;
+                const float r = lo ? 1.0f / plo[e + c < 9 && e + c > 0 ? e + c : 1] : rp_inf;
+                u = div_rn(__builtin_fmaf(-0.5f, u, w[c]), p, r);
+            }
         }
         carry = u;
     }
-    float v[SEG];
-    float last = seg_forward<SEG>(y, yl, yr, dx, carry, i0, nt, p_inf, plo, lane0, v);
+    float last = carry;
+    {
+        uint32_t mn = ~0u;
+#pragma unroll
+        for (int c = 0; c < SEG; ++c) {
+            const bool lo = c < 9 && lane0;
+            const float p = lo ? plo[c < 9 ? c : 0] : p_inf;
+            const float r = lo ? 1.0f / plo[c < 9 && c > 0 ? c : 1] : rp_inf;
+            float un = div_rn(__builtin_fmaf(-0.5f, last, v[c]), p, r);
+            if (c == 0) un = lane0 ? 0.0f : un;  // u_0 = 0
+            last = un;
+            v[c] = (i0 + c <= nt - 2) ? un : 0.0f;
+            const uint32_t b = mag_bits(v[c]);
+            mn = b < mn ? b : mn;
+        }
+        bad = (bad || mn < FAST_ULO) && i0 <= nt - 2;
+    }
     // lanes with i0 > nt-2 hold no u values; their carries need not agree
     for (;;) {
         const float want = from_left(last);
-        const bool redo = lane > 0 && i0 <= nt - 2 && bits_differ(carry, want);
+        const bool redo = bad || (lane > 0 && i0 <= nt - 2 && bits_differ(carry, want));
         if (!any_lane(redo)) break;
         if (redo) {
-            carry = want;
+            if (lane > 0) carry = want;
+            bad = false;
             last = seg_forward<SEG>(y, yl, yr, dx, carry, i0, nt, p_inf, plo, lane0, v);
         }
     }
@@ -463,25 +552,32 @@ __global__ __launch_bounds__(64 * NW) void k_spline_seg(const float *__restrict_
     }
 
     // ---- output ------------------------------------------------------------
-    const int c = 4 * (lane & 7);
     if (MODE == 0) {
-        // 16 samples per pass: lane row = (y_k, h*y2_k) pairs, 32 floats
+        // per pass the whole segments of RP lanes, (y_k, h*y2_k) pairs: 8 KB that
+        // are contiguous in the table, so that its lines are written whole
+        constexpr int RP = 1024 / SEG, PITCH = 2 * SEG + 4;
+        static_assert(RP * PITCH <= 64 * SPL_PITCH, "a pass fits the wave's tile");
         const float h = (1.0f / 6.0f) * (dx * dx);
         float *tab = static_cast<float *>(outp) + ch * (int64_t)(2 * (nt + 1));
+        float *W = &Sw[0][0];
+        const int wl = lane & 63;
+        __syncthreads();  // neighbours have read their rows
 #pragma unroll
-        for (int hh = 0; hh < SEG / 16; ++hh) {
-            __syncthreads();  // staging tile free
+        for (int ps = 0; ps < 64 / RP; ++ps) {
+            if (wl / RP == ps) {
+                float *row = W + (wl % RP) * PITCH;
 #pragma unroll
-            for (int j = 0; j < 16; j += 2)
-                *reinterpret_cast<float4 *>(&S[lane][2 * j]) =
-                    make_float4(y[16 * hh + j], h * v[16 * hh + j], y[16 * hh + j + 1],
-                                h * v[16 * hh + j + 1]);
-            __syncthreads();
+                for (int j = 0; j < SEG; j += 2)
+                    *reinterpret_cast<float4 *>(row + 2 * j) =
+                        make_float4(y[j], h * v[j], y[j + 1], h * v[j + 1]);
+            }
+            tile_sync();
 #pragma unroll
             for (int q = 0; q < 8; ++q) {
-                const int r = row0 + 8 * q + ((lane & 63) >> 3);
-                const int f = 2 * (r * SEG + 16 * hh) + c;  // float index in the row
-                const float4 w = *reinterpret_cast<const float4 *>(&S[r][c]);
+                const int idx = 256 * q + 4 * wl;
+                const float4 w = *reinterpret_cast<const float4 *>(W + idx / (2 * SEG) * PITCH +
+                                                                   idx % (2 * SEG));
+                const int f = 2 * (row0 + RP * ps) * SEG + idx;  // float index in the row
                 if (f + 4 <= 2 * nt) {
                     F4u o{{w.x, w.y, w.z, w.w}};
                     *reinterpret_cast<F4u *>(tab + f) = o;
@@ -492,12 +588,14 @@ __global__ __launch_bounds__(64 * NW) void k_spline_seg(const float *__restrict_
                         if (f + e < 2 * nt) tab[f + e] = e4[e];
                 }
             }
+            tile_sync();
         }
         if (lane0) {
             tab[2 * nt] = 0.0f;
             tab[2 * nt + 1] = 0.0f;
         }
     } else {
+        const int c = 4 * (lane & 7);
         float *y2 = static_cast<float *>(outp) + ch * (int64_t)nt;
 #pragma unroll
         for (int t = 0; t < SEG / 32; ++t) {

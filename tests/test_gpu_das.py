@@ -137,6 +137,45 @@ def test_spline_prefilter_bitwise(nt, data):
     assert np.all(t[:, nt] == 0)
 
 
+@pytest.mark.parametrize("nt", [2, 33, 64, 513, 2048, 2049, 4096, 4097, 9000])
+@pytest.mark.parametrize("dt", [2.0 ** -41, 2.0 ** -40, 2.5e-8, 1.0, 1.5])
+def test_spline_division_range(nt, dt):
+    """The table's bits, signs of zeros included, on both sides of every limit
+    of the sweep's short divisions: samples and steps just inside and outside,
+    decays through denormals, infinities and NaN; against the sweep of one
+    lane per channel, whose divisions are the compiler's."""
+    import torch
+    from pycbf_amd.gpu import _engine as E
+    print(f"spline division range nt={nt} dt={dt}", flush=True)
+    rng = np.random.default_rng(nt)
+    rf = rng.standard_normal((48, nt)).astype(np.float32)
+    for c, (lo, hi) in enumerate([(-46, 39), (-47, 40), (-60, 60), (-126, 100)]):
+        rf[8 * c:8 * c + 8] *= (2.0 ** rng.integers(lo, hi, (8, nt))).astype(np.float32)
+    rf[32:36] *= 1e-30
+    rf[36:40, nt // 3:] = 0.0
+    rf[36:40, nt // 2:] *= -1.0
+    rf[40:44, nt // 2] = np.inf
+    rf[44:, nt // 3] = np.nan
+    dev = torch.device("cuda")
+    x = torch.as_tensor(rf, device=dev)
+    wsb = E.lib.pycbf_spline_workspace_bytes(48, nt)
+    tabs = []
+    try:
+        for seg in ("1", "0"):
+            os.environ["PYCBF_SPLINE_SEG"] = seg
+            need = max(wsb, E.lib.pycbf_spline_workspace_bytes(48, nt))
+            ws = torch.empty(need, dtype=torch.uint8, device=dev)
+            tab = torch.empty((48, nt + 1, 2), dtype=torch.float32, device=dev)
+            E.check(E.lib.pycbf_spline_coefs(E.ptr(x), 48, nt, float(dt), E.ptr(tab), E.ptr(ws),
+                                             need, E.stream_of(dev)), "coefs")
+            tabs.append(tab.cpu().numpy())
+    finally:
+        del os.environ["PYCBF_SPLINE_SEG"]
+    nan = np.isnan(tabs[1])
+    assert np.array_equal(np.isnan(tabs[0]), nan)
+    assert np.array_equal(tabs[0].view(np.uint32)[~nan], tabs[1].view(np.uint32)[~nan])
+
+
 @pytest.mark.parametrize("sumtype", ["none", "tx_only", "rx_only", "tx_and_rx"])
 @pytest.mark.parametrize("interp,kind,usf", KINDS, ids=[k[1] + str(k[2]) for k in KINDS])
 def test_sumtypes_match_oracle(small, sumtype, interp, kind, usf):
