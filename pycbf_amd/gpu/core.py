@@ -204,9 +204,8 @@ class TabbedBeamformer(Tabbed, GPUBeamformer):
         # channel, or per eighth of the channels): it runs over copies whose
         # pixel columns are in that order (contiguous loads per wave), and its
         # image is scattered back to the pixels' own.
-        perm = self._delay_order()
-        self._perm = self._to_dev(perm, dtype=_torch().int32)
-        self._order = self._to_dev(perm, dtype=_torch().int64)
+        self._order = self._to_dev(self._delay_order(), dtype=_torch().int64)
+        self._perm = self._order.to(_torch().int32)
         self._otabs = tuple(t.index_select(1, self._order).contiguous()
                             for t in (self._tautx, self._apodtx, self._taurx, self._apodrx))
         self._obuf = None
