@@ -22,9 +22,9 @@
 // about three lines per gather that the waves in flight must cover.
 // One frame of 75 x 128 x 4096 onto 512 x 512, cubic: 1.84 -> 0.70 ms (the
 // gather with transmit delays in registers before it: 0.48 T wave-level VALU
-// instructions at 30 per sample, and no dropped elements); 31 x 128 x 2048 onto 256 x 256, k-order:
-// 700 -> 117 us (staged through LDS, one barrier per channel, before);
-// 15 x 96 x 2048, linear per-receive images: 248 -> 75 us.
+// instructions at 30 per sample, and no dropped elements); 31 x 128 x 2048 onto
+// 256 x 256, k-order: 700 -> 117 us (staged through LDS, one barrier per
+// channel, before); 15 x 96 x 2048, linear per-receive images: 248 -> 75 us.
 //
 // The frames' sums stay in registers.  tx_and_rx adds the waves' sums in LDS
 // in a fixed order and stores the image once, with no clear and no atomics.
@@ -334,7 +334,8 @@ __device__ __forceinline__ void wave_sweep(const DasArgs &A, const WaveArgs &W, 
 #pragma unroll
         for (int w = 0; w < WAVE_IB / 64; ++w) {
             const int fl = (w * 64 + lane < n) ? s_flag[w * 64 + lane] : 2;
-            const uint64_t m = __ballot((SUM == WS_NONE) ? (w * 64 + lane < n) : (fl & 1) != 0) & share.pat;
+            const uint64_t m =
+                __ballot((SUM == WS_NONE) ? (w * 64 + lane < n) : (fl & 1) != 0) & share.pat;
             mask[w] = ((uint64_t)__builtin_amdgcn_readfirstlane((uint32_t)(m >> 32)) << 32) |
                       (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)m);
             unit = unit && __all((fl & 2) != 0);

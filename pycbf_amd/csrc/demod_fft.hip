@@ -502,7 +502,8 @@ __device__ __forceinline__ void fft_regs(float2 (&v)[P], float2 *B,
 // per butterfly 280 us against 485 when the compiler hoists (spills) them.
 // 32 workgroups per CU: 16 cost 175 us at n = 2048, 64 the same as 32.
 template <int P1, int P2>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void k_demod_regs(DemodFftArgs a)
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2)))
+void k_demod_regs(DemodFftArgs a)
 {
     constexpr int PM = P1 > P2 ? P1 : P2;
     constexpr int KPL = P2 / 2;  // kept bins per lane: m <= L / 2

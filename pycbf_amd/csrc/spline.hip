@@ -2,8 +2,8 @@
 // reads with one load per sample.
 //
 //  * k_spline_seg (nt <= 32768): natural cubic spline (tie_knots1D_fixed,
-//    pycbf/cpu/pycbf.c:114-166), one to eight waves per channel, each lane sweeping a
-//    segment from a verified carry; bit-identical second derivatives.
+//    pycbf/cpu/pycbf.c:114-166), one to eight waves per channel, each lane
+//    sweeping a segment from a verified carry; bit-identical second derivatives.
 //  * k_spline (longer channels): the same spline, one wave owns 64 channels;
 //    32-sample tiles are staged through LDS so that global loads/stores stay
 //    coalesced while each lane runs its channel's sequential recurrence in the
@@ -248,7 +248,8 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3))) void k_
 // Global memory is touched once per sample: the channel is read in coalesced
 // 64 x 32 tiles (row l = 32 samples of lane l's segment) and transposed
 // through one LDS tile; the table goes back by whole segments, the second
-// derivatives by tiles.  Compared with k_spline there is no scratch round trip and no second read of the channel.
+// derivatives by tiles.  Compared with k_spline there is no scratch round trip
+// and no second read of the channel.
 constexpr int SEG_WARM = 32;  // warm-up length of both sweeps (samples)
 
 // Fills u_{i0+c} (c < SEG) from the exact or guessed carry u = u_{i0-1}.
