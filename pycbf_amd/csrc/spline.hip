@@ -252,64 +252,65 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3))) void k_
 // and no second read of the channel.
 constexpr int SEG_WARM = 32;  // warm-up length of both sweeps (samples)
 
-// Fills u_{i0+c} (c < SEG) from the exact or guessed carry u = u_{i0-1}.
-// y = the lane's samples, yl = y_{i0-1}, yr = y_{i0+SEG}.  u values with
-// index > nt-2 are stored as 0 (the back substitution starts at y2_{nt-1}=0).
-// Returns u_{i0+SEG-1} as seen by the right neighbour.
-template <int SEG>
-__device__ __forceinline__ float seg_forward(const float (&y)[SEG], float yl, float yr, float dx,
-                                             float u, int i0, int nt, float p_inf,
-                                             const float (&plo)[9], bool lane0, float (&v)[SEG])
+// x / d.  RECIP: in double from r = 1 / d, which rounds to the float quotient:
+// the product is within 2^-52 of it, and for d <= 2 a quotient of two floats,
+// subnormal ones included, is an exact double or at least 2^-49 from the
+// midpoint of two floats; the signs of zeros, infinities and NaN are the
+// division's.  Three operations against eleven, one of them a quarter-rate
+// reciprocal.
+template <bool RECIP>
+__device__ __forceinline__ float quot(float x, float d, double r)
 {
-    // opaque copies: this sweep runs for few lanes, and what it shares with the
-    // fast one is not to be held in registers for it
+    return RECIP ? (float)((double)x * r) : x / d;
+}
+
+// the divisors of the sweep and their reciprocals
+struct SplineDiv {
+    float dx, dx2, p_inf;
+    double rdx, rdx2, rp_inf;
+};
+
+// g_{i0+c} (c < SEG) of y = the lane's samples, yl = y_{i0-1}, yr = y_{i0+SEG}
+template <int SEG, bool RECIP>
+__device__ __forceinline__ void seg_rhs(const float (&y)[SEG], float yl, float yr,
+                                        const SplineDiv &D, float (&v)[SEG])
+{
+    // opaque copies: a repeated sweep computes these again for a few lanes, and
+    // what it shares with the first is not to be held in registers for it
     float yc = y[0];
     asm volatile("" : "+v"(yc));
-    float d_prev = (yc - yl) / dx;
+    float d_prev = quot<RECIP>(yc - yl, D.dx, D.rdx);
 #pragma unroll
     for (int c = 0; c < SEG; ++c) {
         float ynext = (c + 1 < SEG) ? y[c + 1] : yr;
         asm volatile("" : "+v"(ynext));
-        const float d = (ynext - yc) / dx;
-        yc = ynext;
-        const float g = 6.0f * (d - d_prev) / (2.0f * dx);
+        const float d = quot<RECIP>(ynext - yc, D.dx, D.rdx);
+        v[c] = quot<RECIP>(6.0f * (d - d_prev), D.dx2, D.rdx2);
         d_prev = d;
+        yc = ynext;
+    }
+}
+
+// Fills u_{i0+c} (c < SEG) from g in v and the exact or guessed carry u =
+// u_{i0-1}.  u values with index > nt-2 are stored as 0 (the back substitution
+// starts at y2_{nt-1}=0).  Returns u_{i0+SEG-1} as seen by the right neighbour.
+template <int SEG, bool RECIP>
+__device__ __forceinline__ float seg_forward(float u, int i0, int nt, const SplineDiv &D,
+                                             const float (&plo)[9], bool lane0, float (&v)[SEG])
+{
+#pragma unroll
+    for (int c = 0; c < SEG; ++c) {
         // p_i = 0.5*y2f[i-1] + 2 differs from p_inf only for i < 9 (lane 0)
-        const float p = (c < 9 && lane0) ? plo[c < 9 ? c : 0] : p_inf;
-        float un = (g - 0.5f * u) / p;
+        const bool lo = c < 9 && lane0;
+        const float p = lo ? plo[c < 9 ? c : 0] : D.p_inf;
+        const double r = lo ? 1.0 / (double)plo[c < 9 && c > 0 ? c : 1] : D.rp_inf;
+        float un = quot<RECIP>(v[c] - 0.5f * u, p, r);
         if (c == 0) un = lane0 ? 0.0f : un;  // u_0 = 0
         u = un;
         v[c] = (i0 + c <= nt - 2) ? u : 0.0f;
     }
     return u;
 }
-
-// x / d from r = 1 / d rounded to nearest, rounded as the division is: two
-// corrections by the exact remainder (P. Markstein, "Computation of elementary
-// functions on the IBM RISC System/6000 processor", 1990: the second starts
-// within one unit in the last place).  Exact remainders need x = +-0 or |x| a
-// factor 2^48 above the smallest float, and |x / d| normal.  Five operations
-// against eleven, one of them a quarter-rate reciprocal.
-__device__ __forceinline__ float div_rn(float x, float d, float r)
-{
-    const float q0 = x * r;
-    const float q1 = __builtin_fmaf(-__builtin_fmaf(q0, d, -x), r, q0);
-    return __builtin_fmaf(-__builtin_fmaf(q1, d, -x), r, q1);
-}
-
-// |v| - 1 in units of the last place: 0 is the largest unsigned and the
-// smallest signed value, NaN a large one of both
-__device__ __forceinline__ uint32_t mag_bits(float v)
-{
-    return (__float_as_uint(v) & 0x7fffffffu) - 1u;
-}
-
-// The inputs that keep every division of the fast sweep in div_rn's range: dx
-// in [2^-40, 1], samples 0 or 2^-46 <= |y| <= 2^40 (so that differences and
-// difference quotients are 0 or >= 2^-93 and g <= 2^124), and u values 0 or
-// >= 2^-96 (they decay through stretches of zeros).
-constexpr uint32_t FAST_YLO = (127u - 46u) << 23, FAST_YHI = (127u + 40u) << 23;
-constexpr uint32_t FAST_ULO = (127u - 96u) << 23;
 
 // y2_{i0+c} = y2f[i0+c] * y2_{i0+c+1} + u_{i0+c}, c = SEG-1 .. 0, in place,
 // from the carry y2_{i0+SEG}.  Returns y2_{i0}.
@@ -349,15 +350,17 @@ __device__ __forceinline__ bool bits_differ(float a, float b)
 // and with 128-byte pieces of every segment per output pass the unaligned rows
 // of the table were written as halves of lines, which L2 no longer joined
 // once the arithmetic was out of the way (9600 x 4096: 134 us before, 147
-// with the cheap divisions alone, 99 with whole-segment passes as well: 4.8
-// TB/s; 153 600 x 4096 1735 -> 1370, 5.5 TB/s; 9600 x 2048 67 -> 43;
-// 3968 x 5000 120 -> 83).  Reading by whole segments as well put each pass's
-// loads behind the last one's: 135 at 9600 x 4096.  Two waves of 32-sample
-// lanes for 2049 .. 4096 samples measured the same on one frame and 1 % slower
-// on sixteen.  k_spline, one lane per channel, waits on its serial chain
-// whatever the channel count: 2106 channels of 4596 samples 1175 us, here 56;
-// 1000 of 20 000 samples 5.2 ms, here 0.10.
-template <int MODE, int SEG, int NW>  // MODE 0: (y, dx^2/6*y2) gather table, 1: y2
+// with cheap divisions alone, 96 with whole-segment passes as well; 153 600 x
+// 4096 1735 -> 1366; 9600 x 2048 67 -> 41; 3968 x 5000 120 -> 79; channels that
+// decay through denormals, 9600 x 2048: 80 -> 57).  Quotients in float, from a
+// rounded reciprocal and two exact remainders, were as fast on noise but need
+// a range, and channels that leave it swept twice (the same: 106).  Reading by whole
+// segments as well put each pass's loads behind the last one's: 135 at
+// 9600 x 4096.  Two waves of 32-sample lanes for 2049 .. 4096 samples measured
+// the same on one frame and 1 % slower on sixteen.  k_spline, one lane per
+// channel, waits on its serial chain whatever the channel count: 2106 channels
+// of 4596 samples 1175 us, here 53; 1000 of 20 000 samples 5.2 ms, here 0.097.
+template <int MODE, int SEG, int NW, bool RECIP>  // MODE 0: (y, dx^2/6*y2) gather table, 1: y2
 __global__ __launch_bounds__(64 * NW) void k_spline_seg(const float *__restrict__ rf, int nt,
                                                         float dx, void *__restrict__ outp)
 {
@@ -441,27 +444,11 @@ __global__ __launch_bounds__(64 * NW) void k_spline_seg(const float *__restrict_
     const float yr = from_right(y[0]);       // y_{i0+SEG}
 
     // ---- forward sweep -----------------------------------------------------
-    // the fast form first, in place: g, then u from it; bad = a division left
-    // the range of div_rn, the lane sweeps again with the divisions themselves
+    // the right-hand sides g, then u from them in place
     float v[SEG];
-    bool bad;
-    const float rdx = 1.0f / dx, dx2 = 2.0f * dx, rdx2 = 1.0f / dx2;
-    {
-        uint32_t mn = mag_bits(yl) < mag_bits(yr) ? mag_bits(yl) : mag_bits(yr);
-        int32_t mx = (int32_t)mag_bits(yl) > (int32_t)mag_bits(yr) ? (int32_t)mag_bits(yl)
-                                                                   : (int32_t)mag_bits(yr);
-        float d_prev = div_rn(y[0] - yl, dx, rdx);
-#pragma unroll
-        for (int c = 0; c < SEG; ++c) {
-            const uint32_t b = mag_bits(y[c]);
-            mn = b < mn ? b : mn;
-            mx = (int32_t)b > mx ? (int32_t)b : mx;
-            const float d = div_rn(((c + 1 < SEG) ? y[c + 1] : yr) - y[c], dx, rdx);
-            v[c] = div_rn(6.0f * (d - d_prev), dx2, rdx2);
-            d_prev = d;
-        }
-        bad = mn < FAST_YLO - 1u || mx > (int32_t)FAST_YHI || !(dx >= 0x1p-40f && dx <= 1.0f);
-    }
+    const SplineDiv D{dx, 2.0f * dx, p_inf, 1.0 / (double)dx, 1.0 / (double)(2.0f * dx),
+                      1.0 / (double)p_inf};
+    seg_rhs<SEG, RECIP>(y, yl, yr, D, v);
     // guess of u_{i0-1}: u = 0 at i0-32, then i = i0-31 .. i0-1 over the left
     // neighbour's last g values
     __syncthreads();  // the samples are read out of the tile
@@ -470,7 +457,6 @@ __global__ __launch_bounds__(64 * NW) void k_spline_seg(const float *__restrict_
         *reinterpret_cast<float4 *>(&S[lane][e]) =
             make_float4(v[SEG - 32 + e], v[SEG - 31 + e], v[SEG - 30 + e], v[SEG - 29 + e]);
     __syncthreads();
-    const float rp_inf = 1.0f / p_inf;
     float carry = 0.0f;
     if (lane > 0) {
         // only lane 1 of a 32-sample segment reaches i < 9 here
@@ -483,39 +469,24 @@ __global__ __launch_bounds__(64 * NW) void k_spline_seg(const float *__restrict_
 #pragma unroll
             for (int c = e == 0 ? 1 : 0; c < 4; ++c) {
                 const bool lo = e + c < 9 && low;
-                const float p = lo ? plo[e + c < 9 ? e + c : 0] : p_inf;
-                const float r = lo ? 1.0f / plo[e + c < 9 && e + c > 0 ? e + c : 1] : rp_inf;
-                u = div_rn(__builtin_fmaf(-0.5f, u, w[c]), p, r);
+                const float p = lo ? plo[e + c < 9 ? e + c : 0] : D.p_inf;
+                const double r = lo ? 1.0 / (double)plo[e + c < 9 && e + c > 0 ? e + c : 1]
+                                    : D.rp_inf;
+                u = quot<RECIP>(w[c] - 0.5f * u, p, r);
             }
         }
         carry = u;
     }
-    float last = carry;
-    {
-        uint32_t mn = ~0u;
-#pragma unroll
-        for (int c = 0; c < SEG; ++c) {
-            const bool lo = c < 9 && lane0;
-            const float p = lo ? plo[c < 9 ? c : 0] : p_inf;
-            const float r = lo ? 1.0f / plo[c < 9 && c > 0 ? c : 1] : rp_inf;
-            float un = div_rn(__builtin_fmaf(-0.5f, last, v[c]), p, r);
-            if (c == 0) un = lane0 ? 0.0f : un;  // u_0 = 0
-            last = un;
-            v[c] = (i0 + c <= nt - 2) ? un : 0.0f;
-            const uint32_t b = mag_bits(v[c]);
-            mn = b < mn ? b : mn;
-        }
-        bad = (bad || mn < FAST_ULO) && i0 <= nt - 2;
-    }
+    float last = seg_forward<SEG, RECIP>(carry, i0, nt, D, plo, lane0, v);
     // lanes with i0 > nt-2 hold no u values; their carries need not agree
     for (;;) {
         const float want = from_left(last);
-        const bool redo = bad || (lane > 0 && i0 <= nt - 2 && bits_differ(carry, want));
+        const bool redo = lane > 0 && i0 <= nt - 2 && bits_differ(carry, want);
         if (!any_lane(redo)) break;
         if (redo) {
-            if (lane > 0) carry = want;
-            bad = false;
-            last = seg_forward<SEG>(y, yl, yr, dx, carry, i0, nt, p_inf, plo, lane0, v);
+            carry = want;
+            seg_rhs<SEG, RECIP>(y, yl, yr, D, v);
+            last = seg_forward<SEG, RECIP>(carry, i0, nt, D, plo, lane0, v);
         }
     }
     const float carry_fwd = carry;
@@ -547,7 +518,8 @@ __global__ __launch_bounds__(64 * NW) void k_spline_seg(const float *__restrict_
         if (redo) {
             // rebuild u from the exact forward carry, then substitute again
             bcarry = want;
-            seg_forward<SEG>(y, yl, yr, dx, carry_fwd, i0, nt, p_inf, plo, lane0, v);
+            seg_rhs<SEG, RECIP>(y, yl, yr, D, v);
+            seg_forward<SEG, RECIP>(carry_fwd, i0, nt, D, plo, lane0, v);
             first = seg_backward<SEG>(v, bcarry, y2f_inf, flo, lane0);
         }
     }
@@ -640,26 +612,35 @@ int spline_seg_len(int32_t nt)
     return 0;
 }
 
+template <int MODE, bool RECIP>
+static void launch_seg(const float *rf, int64_t nch, int nt, float dt, void *out, hipStream_t s)
+{
+    const dim3 grid((unsigned)nch);
+    if (nt <= 64 * 32)
+        hipLaunchKernelGGL((k_spline_seg<MODE, 32, 1, RECIP>), grid, dim3(64), 0, s, rf, nt, dt, out);
+    else if (nt <= 64 * 64)
+        hipLaunchKernelGGL((k_spline_seg<MODE, 64, 1, RECIP>), grid, dim3(64), 0, s, rf, nt, dt, out);
+    else if (nt <= 2 * 64 * 64)
+        hipLaunchKernelGGL((k_spline_seg<MODE, 64, 2, RECIP>), grid, dim3(128), 0, s, rf, nt, dt, out);
+    else if (nt <= 4 * 64 * 64)
+        hipLaunchKernelGGL((k_spline_seg<MODE, 64, 4, RECIP>), grid, dim3(256), 0, s, rf, nt, dt, out);
+    else
+        hipLaunchKernelGGL((k_spline_seg<MODE, 64, 8, RECIP>), grid, dim3(512), 0, s, rf, nt, dt, out);
+}
+
 template <int MODE>
 static int launch_spline(const float *rf, int64_t nch, int32_t nt, float dt, float *uscr,
                          void *out, hipStream_t s)
 {
     if (nch <= 0 || nt <= 0) return 0;
     if (nt > SPL_MAX_NT) return fail(1, "spline: nt %d exceeds %d samples", nt, SPL_MAX_NT);
-    const dim3 grid((unsigned)nch);
     if (!spline_segments())
         hipLaunchKernelGGL(k_spline<MODE>, dim3((unsigned)((nch + 63) / 64)), dim3(64), 0, s, rf,
                            nch, (int)nt, dt, uscr, out);
-    else if (nt <= 64 * 32)
-        hipLaunchKernelGGL((k_spline_seg<MODE, 32, 1>), grid, dim3(64), 0, s, rf, (int)nt, dt, out);
-    else if (nt <= 64 * 64)
-        hipLaunchKernelGGL((k_spline_seg<MODE, 64, 1>), grid, dim3(64), 0, s, rf, (int)nt, dt, out);
-    else if (nt <= 2 * 64 * 64)
-        hipLaunchKernelGGL((k_spline_seg<MODE, 64, 2>), grid, dim3(128), 0, s, rf, (int)nt, dt, out);
-    else if (nt <= 4 * 64 * 64)
-        hipLaunchKernelGGL((k_spline_seg<MODE, 64, 4>), grid, dim3(256), 0, s, rf, (int)nt, dt, out);
     else if (nt <= 8 * 64 * 64)
-        hipLaunchKernelGGL((k_spline_seg<MODE, 64, 8>), grid, dim3(512), 0, s, rf, (int)nt, dt, out);
+        // the reciprocal form's proof needs divisors up to 2 (and they include 2 dt)
+        dt <= 1.0f ? launch_seg<MODE, true>(rf, nch, (int)nt, dt, out, s)
+                   : launch_seg<MODE, false>(rf, nch, (int)nt, dt, out, s);
     else
         hipLaunchKernelGGL(k_spline<MODE>, dim3((unsigned)((nch + 63) / 64)), dim3(64), 0, s, rf,
                            nch, (int)nt, dt, uscr, out);

@@ -140,10 +140,10 @@ def test_spline_prefilter_bitwise(nt, data):
 @pytest.mark.parametrize("nt", [2, 33, 64, 513, 2048, 2049, 4096, 4097, 9000])
 @pytest.mark.parametrize("dt", [2.0 ** -41, 2.0 ** -40, 2.5e-8, 1.0, 1.5])
 def test_spline_division_range(nt, dt):
-    """The table's bits, signs of zeros included, on both sides of every limit
-    of the sweep's short divisions: samples and steps just inside and outside,
-    decays through denormals, infinities and NaN; against the sweep of one
-    lane per channel, whose divisions are the compiler's."""
+    """The table's bits, signs of zeros included, for steps on both sides of the
+    reciprocal form's limit and samples over the whole range: decays through
+    denormals, infinities and NaN; against the sweep of one lane per channel,
+    whose divisions are the compiler's."""
     import torch
     from pycbf_amd.gpu import _engine as E
     print(f"spline division range nt={nt} dt={dt}", flush=True)
