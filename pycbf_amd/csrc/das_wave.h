@@ -111,7 +111,9 @@ __device__ __forceinline__ uint32_t wave_off(int j, float jf, float bytes)
     return __float_as_uint(__builtin_fmaf(jf, bytes, WAVE_OFF_BIAS));
 }
 
-// INSIDE: every lane's x is known to lie on the trace
+// INSIDE: every lane's x is known to lie on the trace, and for nearest also to
+// round to one of its entries (a last sample time that float rounding has moved
+// up by half a sample or more rounds to the entry after them)
 template <int GK, int MODE, bool EXACT, bool INSIDE>
 __device__ __forceinline__ WavePos wave_pos(const DasArgs &A, float nhalf, float x)
 {
@@ -291,6 +293,10 @@ __device__ __forceinline__ void wave_sweep(const DasArgs &A, const WaveArgs &W, 
     const bool inner_tx = W.inner_tx != 0;
     const int no = inner_tx ? A.nrx : A.ntx;
     const bool drop = A.thresh > 0.0f;  // a zero (or NaN) weight then never contributes
+    // nearest: whether the last sample time rounds to an entry, as then every
+    // earlier one does (quotients are monotone in the time)
+    const bool last_in =
+        GK != GK_NEAREST || wave_pos<GK, MODE, EXACT, false>(A, W.nhalf, A.tmax).in;
     float *s_tau = sm;
     float *s_wgt = sm + W.ib * 64;
     // this lane's column of s_tau as an LDS address the compiler holds in one
@@ -443,7 +449,7 @@ __device__ __forceinline__ void wave_sweep(const DasArgs &A, const WaveArgs &W, 
             };
             if (SUM == WS_NONE || __any(to == to)) {
                 // every sample of the wave on the trace: no clamps, no selects
-                const bool inside = SUM != WS_NONE && unit &&
+                const bool inside = SUM != WS_NONE && unit && last_in &&
                                     __all(lo + to >= A.t0 && hi + to <= A.tmax);
                 if (inside)
                     sweep(std::integral_constant<int, SUM == WS_NONE ? 1 : 2>());

@@ -72,6 +72,39 @@ def test_wave_gather_matches_oracle(ntx, nrx, npx, nfr, t0, unit, interp, usf, m
             assert_close_to_peak(got, ref.reshape(got.shape), 1e-5, sumtype)
 
 
+def _last_quotient(t0, nt, usf):
+    """(tmax - t0) / dt of the (upsampled) trace in float32, and its entries."""
+    f = np.float32
+    t0, dt = f(t0), f(DT)
+    return float((f(t0 + dt * f(nt - 1)) - t0) / f(dt / f(usf))), usf * (nt - 1) + 1
+
+
+@pytest.mark.parametrize("nfr", [None, 4])
+@pytest.mark.parametrize("t0,nt,usf,past", [(0.5, 60, 1, 0.5), (0.5, 69, 1, 1.0), (0.05, 500, 16, 0.5)])
+def test_nearest_at_a_last_sample_time_that_rounds_past_the_trace(t0, nt, usf, past, nfr):
+    """A start so late that float32 moves the last sample time up by half a
+    sample (past 0.5: the reciprocal quotients) or a whole one (past 1: the
+    division): a delay there, in waves that lie on the trace as a whole, selects
+    no sample.  Nearest picks samples, so the bar is the sum's own rounding."""
+    q, n = _last_quotient(t0, nt, usf)
+    assert n - 1 + past <= q < n - 0.5 + past
+    rng = np.random.default_rng(nt)
+    ntx, nrx, npx = 9, 10, 130
+    last = np.float32(t0) + np.float32(DT) * np.float32(nt - 1)
+    tautx = np.repeat(np.linspace(t0, last, npx, dtype=np.float32)[None], ntx, axis=0)
+    tautx[:, ::4] = last
+    assert tautx.min() >= np.float32(t0) and tautx.max() == last
+    tabs = (tautx, np.ones((ntx, npx), np.float32), np.zeros((nrx, npx), np.float32),
+            np.ones((nrx, npx), np.float32))
+    rf = rng.standard_normal((nfr or 1, ntx, nrx, nt)).astype(np.float32)
+    for sumtype in ("tx_and_rx", "tx_only", "rx_only"):
+        print(f"late nearest t0={t0} nt={nt} usf={usf} nfr={nfr} {sumtype}", flush=True)
+        got = _beamformer(tabs, t0, nt, {"kind": "nearest", "usf": usf}, sumtype)(rf if nfr else rf[0])
+        ref = oracle.das_tabbed(rf if nfr else rf[0], t0, DT, *tabs, kind="nearest", usf=usf, sumtype=sumtype)
+        assert not ref[..., ::4].any()
+        assert_close_to_peak(got, ref, 1e-5, sumtype)
+
+
 @pytest.mark.parametrize("thresh", [0.0, 1e-2, 1.5])
 @pytest.mark.parametrize("nfr", [None, 4])
 @pytest.mark.parametrize("kind", ["cubic", "korder_cubic"])
