@@ -25,6 +25,7 @@
 #include <math.h>
 
 #include <algorithm>
+#include <cmath>
 #include <type_traits>
 #include <vector>
 
@@ -395,6 +396,14 @@ int pycbf_batch_create(const pycbf_batch_req *reqs, int nreq, pycbf_batch **out)
         P.ch_off.push_back(chans);
         chans += (int64_t)q.ntx * q.nrx;
         P.reqs.push_back(q);
+        // No time lies on a trace whose start (or end) is no finite number, and the
+        // gather's row offsets are formed from the quotient by dt: the request keeps
+        // its zeros through a threshold that no weight reaches.
+        const float tmax = q.t0 + q.dt * (float)(P.nt - 1);
+        if (!std::isfinite(q.t0) || std::isnan(tmax)) {
+            P.reqs.back().t0 = 0.0f;
+            P.reqs.back().thresh = INFINITY;
+        }
     }
     if (!das_contig)
         return fail(PYCBF_EINVAL, "DAS outputs must be contiguous, in request order");

@@ -88,10 +88,11 @@ enum WaveSum { WS_BOTH = 0, WS_SEP = 1, WS_NONE = 2 };
 enum WaveMode { WM_DIV = 0, WM_RECIP = 1, WM_RECIP0 = 2 };
 
 // The mode for a trace of nsrc entries; host only.  The reciprocal modes do not
-// clamp the knot index, so the last sample time itself must select a knot.
+// clamp the knot index, so the last sample time itself must select a knot (a
+// quotient that is no number does not).
 inline int wave_mode_of(float t0, float dt, float rdt, float tmax, int64_t nsrc)
 {
-    if (nsrc > WAVE_FLOAT_NSRC || !((int)((tmax - t0) / dt) <= nsrc - 1)) return WM_DIV;
+    if (nsrc > WAVE_FLOAT_NSRC || !((tmax - t0) / dt < (float)nsrc)) return WM_DIV;
     if (rdt != 1.0f / dt || !recip_division_exact(dt)) return WM_DIV;
     return t0 == 0.0f ? WM_RECIP0 : WM_RECIP;
 }

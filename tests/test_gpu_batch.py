@@ -155,3 +155,23 @@ def test_batch_gather_branches(t0, thresh):
         for bf, v, o in zip(singles, batch.rf_views, batch.outputs):
             ref = bf(v, out_as_numpy=False).reshape(o.shape)
             assert float((o - ref).abs().max()) <= 1e-5 * float(ref.abs().max()), (tile, rchunk, tuple(o.shape))
+
+
+@pytest.mark.parametrize("t0", [float("nan"), float("inf"), -float("inf")])
+def test_batch_without_a_finite_trace_start(t0):
+    """No time lies on a trace that starts nowhere: zero images, from few and
+    from many transmits."""
+    import torch
+    from pycbf_amd import sim
+    from pycbf_amd.gpu.batch import BatchRequest, RaggedBatch
+    reqs = []
+    for ntx, nrx, nx, nz in ((2, 20, 5, 7), (9, 8, 12, 9)):
+        _, _, pnts = sim.grid(nx, nz, (-2e-3, 2e-3), (2e-3, 7e-3))
+        p = sim.pw_synthetic(np.radians(np.linspace(-9, 9, ntx)), sim.linear_array(nrx), pnts)
+        reqs.append(BatchRequest(params=p, gridshape=(nx, nz)))
+    print(f"ragged batch t0={t0}", flush=True)
+    batch = RaggedBatch(reqs, nt=500, dt=1.0 / sim.FS, t0=t0)
+    batch.rf_all.normal_()
+    batch.run()
+    torch.cuda.synchronize()
+    assert not any(bool(o.any()) for o in batch.outputs)
