@@ -512,7 +512,8 @@ __global__ __launch_bounds__(256) void k_unit_delays(BwdArgs A, float *__restric
 // A contribution becomes an integer by adding 1.5 2^52 to it in double, exact to
 // the last bit kept while it stays below 2^51 (MAGIC; two instructions and an
 // integer subtraction, against about ten for the conversion): images of 256
-// pixels and more, whose bins leave that much room.
+// pixels and more, whose bins leave that much room, on time axes that float32
+// resolves (launch_rf_ch_src).
 // 31 x 128 x 4096 onto 256 x 256, cubic, tables: 606 -> 433 us; 16 x 64 x
 // 2048 onto 192 x 256, linear, geometry: 222 -> 74 us and 11 for its table.
 enum RfSource { RF_TABLES = 0, RF_UNIT = 1, RF_GEOM = 2 };
@@ -1168,9 +1169,15 @@ int bwd_per_channel(int gk, const BwdArgs &a, bool &yes)
 template <int GK, int GEO, bool FD, int SRC>
 static int launch_rf_ch_src(const BwdArgs &a, int64_t nch, size_t lds, hipStream_t s)
 {
-    // the magic conversion needs contributions below 2^51: bwd_scale leaves them
-    // below 2^(60 - per_bin), per_bin >= 10
-    if (a.np >= 256)
+    // The magic conversion needs contributions below 2^51.  bwd_scale leaves
+    // gout times weight below 2^(60 - per_bin), per_bin >= 10 from 256 pixels on;
+    // the interpolation weights must not double that.  Knot times are rounded to
+    // u = 2^-23 max(|t0|, |tmax|) or better and a position to its knots is off by
+    // 4 u at most: with 16 u <= dt the weights are of a position in
+    // [-1/4, 5/4], 1.96 at most ((5/4)^3 of the Hermite kinds).  (Half a second
+    // into a trace of 31 ns samples they reach 7.)
+    const float u = 0x1p-23f * std::max(fabsf(a.t0), fabsf(a.tmax));
+    if (a.np >= 256 && (GK == GK_NEAREST || 16.0f * u <= a.dt))
         hipLaunchKernelGGL((k_das_bwd_rf_ch<GK, GEO, FD, SRC, true>), dim3((unsigned)nch),
                            dim3(1024), lds, s, a);
     else

@@ -326,3 +326,28 @@ def test_adjoint_at_tile_and_block_edges(kind, ntx, nrx, npx, nfr):
     assert np.max(np.abs(out - ref_out)) <= 1e-4 * np.max(np.abs(ref_out))
     for name, a, b in zip(NAMES, g, gr):
         assert np.max(np.abs(a - b)) <= 1e-4 * np.max(np.abs(b)), name
+
+
+@pytest.mark.parametrize("kind", ["cubic", "akima", "korder_cubic"])
+def test_rf_adjoint_where_float32_does_not_resolve_the_samples(kind):
+    """Half a second into a trace of 31 ns samples float32 times lie 1.9 samples
+    apart, and interpolation weights reach 5 (cubic) and 7 (Akima): the bins'
+    conversion has to hold them.  Equal upstream gradients just below the scale's
+    next power of two, on 256 pixels.  The channel-data gradient is the transpose
+    of the forward, which rounds the same times: the bar is 1e-5 of the sum of the
+    transpose identity's terms (rounding of each)."""
+    import torch
+    from pycbf_amd.gpu.autograd import das_tabbed
+    nt, t0, dt = 120, 0.5, 2.0 ** -24 / 1.92
+    late = [t0 + k * 2.0 ** -24 for k in (13, 25)]  # 1.92 samples from one of their knots
+    tautx = np.repeat(np.float32([late]), 128, axis=0).reshape(1, 256)
+    one = np.ones((1, 256), np.float32)
+    d = lambda a: torch.as_tensor(a, device="cuda")  # noqa: E731
+    rf = d(np.random.default_rng(6).standard_normal((1, 1, nt)).astype(np.float32)).requires_grad_()
+    out = das_tabbed(rf, d(tautx), d(one), d(0.0 * one), d(one), t0, dt, kind, "tx_and_rx", 1e-2,
+                     k=8 if kind == "korder_cubic" else None)
+    assert float(out.detach().abs().min()) > 0
+    (grf,) = torch.autograd.grad(1.99 * out.sum(), [rf])
+    lhs = 1.99 * float(out.detach().double().sum())
+    terms = rf.detach().double() * grf.double()
+    assert abs(lhs - float(terms.sum())) <= 1e-5 * float(terms.abs().sum()), (lhs, float(terms.sum()))
