@@ -356,6 +356,10 @@ __device__ __forceinline__ void wave_sweep(const DasArgs &A, const WaveArgs &W, 
             elem_eval<GEO>(A, !inner_tx, o, p, pv, to, wo);
             if (!act || (drop && !(wo != 0.0f && wo == wo))) to = NAN;
             if (unit && !(fabsf(wo) >= A.thresh)) to = NAN;
+            // an infinite outer weight goes to every sample: times a sum it would
+            // be NaN where no sample counts, or where the sum has lost a sign
+            const bool whole = unit && (GEOM || SUM == WS_NONE ||
+                                        __all(!(to == to) || fabsf(wo) < INFINITY));
             float part[FC];
 #pragma unroll
             for (int f = 0; f < FC; ++f) part[f] = 0.0f;
@@ -450,17 +454,17 @@ __device__ __forceinline__ void wave_sweep(const DasArgs &A, const WaveArgs &W, 
             };
             if (SUM == WS_NONE || __any(to == to)) {
                 // every sample of the wave on the trace: no clamps, no selects
-                const bool inside = SUM != WS_NONE && unit && last_in &&
+                const bool inside = SUM != WS_NONE && whole && last_in &&
                                     __all(lo + to >= A.t0 && hi + to <= A.tmax);
                 if (inside)
                     sweep(std::integral_constant<int, SUM == WS_NONE ? 1 : 2>());
-                else if (unit)
+                else if (whole)
                     sweep(std::integral_constant<int, 1>());
                 else
                     sweep(std::integral_constant<int, 0>());
             }
             if (SUM == WS_NONE) continue;
-            if (!GEOM && unit) {
+            if (!GEOM && whole) {
 #pragma unroll
                 for (int f = 0; f < FC; ++f) part[f] *= (to == to) ? wo : 0.0f;
             }

@@ -105,6 +105,39 @@ def test_nearest_at_a_last_sample_time_that_rounds_past_the_trace(t0, nt, usf, p
         assert_close_to_peak(got, ref, 1e-5, sumtype)
 
 
+@pytest.mark.parametrize("interp", [{"kind": "cubic"}, {"kind": "linear"}, {"kind": "korder_cubic", "k": 8}],
+                         ids=lambda i: i["kind"])
+@pytest.mark.parametrize("ntx", [3, 9])
+@pytest.mark.parametrize("on", ["tx", "rx"])
+def test_infinite_weights_on_one_axis(on, ntx, interp, monkeypatch):
+    """Weights of one on one axis and infinite ones on the other, where no sample
+    lies on the trace (nothing is added) and where some do (infinite, or NaN where
+    the signs differ): the infinities, NaN and finite pixels of the kernel that
+    adds each sample by itself."""
+    rng = np.random.default_rng(8)
+    nrx, npx, nt = 12, 140, 200
+    span = np.float32(nt * DT)
+    tau = {"tx": rng.uniform(0, 0.4, (ntx, npx)).astype(np.float32) * span,
+           "rx": rng.uniform(0, 0.4, (nrx, npx)).astype(np.float32) * span}
+    apod = {"tx": np.ones((ntx, npx), np.float32), "rx": np.ones((nrx, npx), np.float32)}
+    apod[on][1, ::7] = np.inf
+    tau[on][1, ::7] += 2 * span   # off the trace
+    apod[on][2, 3::7] = np.inf    # on it
+    tabs = (tau["tx"], apod["tx"], tau["rx"], apod["rx"])
+    rf = rng.standard_normal((ntx, nrx, nt)).astype(np.float32)
+    for sumtype in ("tx_and_rx", "tx_only", "rx_only"):
+        print(f"infinite {on} weights ntx={ntx} {interp['kind']} {sumtype}", flush=True)
+        got = _beamformer(tabs, 0.0, nt, interp, sumtype)(rf)
+        monkeypatch.setenv("PYCBF_DAS_PLAIN", "1")
+        ref = _beamformer(tabs, 0.0, nt, interp, sumtype)(rf)
+        monkeypatch.delenv("PYCBF_DAS_PLAIN")
+        fin = np.isfinite(ref)
+        assert fin[..., ::7].all() and not fin.all()
+        assert np.array_equal(got[~fin], ref[~fin], equal_nan=True)
+        assert np.isfinite(got[fin]).all()
+        assert_close_to_peak(got[fin], ref[fin], 1e-5, sumtype)
+
+
 @pytest.mark.parametrize("thresh", [0.0, 1e-2, 1.5])
 @pytest.mark.parametrize("nfr", [None, 4])
 @pytest.mark.parametrize("kind", ["cubic", "korder_cubic"])
