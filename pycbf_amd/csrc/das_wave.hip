@@ -16,11 +16,58 @@ int wave_launch_sample(int gk, const DasArgs &a, const WaveArgs &w, int sum, int
     return wave_sum<GK_LINEAR>(sum, fc, mode, a, w, grid, nw, lds, s);
 }
 
+// Four frames of the gather table, the most that one pass reads.
+static int64_t pass_table_bytes(const DasArgs &a)
+{
+    return (int64_t)a.ntx * a.nrx * a.ch_stride * 4 * 4;
+}
+constexpr int64_t BIG_TABLE = (int64_t)96 << 20;
+
+// Whether each XCD takes every eighth outer element over all tiles, so that a
+// channel's row enters one L2 only, instead of runs of tiles over all elements.
+// Four or more frames; the outer axis has to give each of the 8 chunks two
+// elements and more.  Times of this order over the other, and over the staged
+// gather (k_das_lds):
+//   tables over 96 MB per pass are pulled again by every XCD: 31 x 128 x 2048 x
+//   200 x 200, k-order, 0.65 - 0.82, 60 x 64 x 2000, linear, 0.46 - 0.65;
+//   smaller ones are not, and the chunks' partial images and idle waves cost
+//   more: 16 x 48 x 800 onto 200 x 200, 16 frames, nearest 2.2 (1.36 of the
+//   staged gather, the other 0.63), 12 x 128 x 1024, nearest, 2.1;
+//   64 tiles and fewer leave the chip short of workgroups, of which this order has
+//   8 times as many: 75 x 32 x 600 onto 1551 pixels, 4 frames, linear, 0.64.
+// Images per element have no partials, and their chunks cost idle waves where
+// the axis is short: 1 x 128 x 1024 onto 20 000 pixels, per transmit, 16
+// frames, 4.9 of the other order (1.87 of the staged gather, the other 0.37).
+static bool wave_slab(int gk, const DasArgs &a, int sum, int no, int ni, int64_t ntiles,
+                      int64_t passes)
+{
+    const bool wide = gk == GK_KORDER || gk == GK_AKIMA;  // 16-byte entries
+    const int64_t table = pass_table_bytes(a);
+    // per-sample outputs: 0.4 - 1 over the geometry and a table beyond one L2, up to
+    // 1.3 over delay tables (40 x 16 x 600, 16 frames), which each XCD reads whole
+    if (sum == WS_NONE) return a.geo && ni >= 2 && no >= 16 && table >= (int64_t)4 << 20;
+    const bool few = no >= 8 && ntiles * (wide ? 1 : passes) <= 64;
+    const bool big = no >= 16 && table >= BIG_TABLE && (a.geo || no >= 48);
+    if (sum == WS_BOTH) return few || big;
+    if (ni == 1) return no >= 16 && passes >= 4 && ntiles > 64;
+    if (few) return true;
+    return wide ? no >= 16 : (a.sumflag == PYCBF_SUM_RX_ONLY ? no >= 32 : big);
+}
+
 bool das_wave_applies(int gk, const DasArgs &a)
 {
     if (gk == GK_LINEAR && a.nsrc < 2) return false;      // reads pairs
     if (gk == GK_NEAREST && a.nsrc > 1 << 22) return false;  // nsrc - 1/2 as a float
     if (a.np > (int64_t)1 << 28) return false;  // 16 threads per pixel within a 32-bit grid
+    // Nearest, sums of many transmits over many frames of a table beyond the L2s:
+    // a sample is little more than its position, which the staged gather shares
+    // among 16 frames and this one among 4 (16 frames of 75 x 40 x 3000 onto 128 x
+    // 128: 474 us staged, 640 here; of 64 x 64 x 2000 onto 100 x 100: 376, 466).  At
+    // 128 tiles and fewer, or few transmits, this one is faster all the same (31 x
+    // 128 x 2048 onto 64 x 64: 0.56 of it).
+    if (gk == GK_NEAREST && a.nfr > 8 && a.sumflag != PYCBF_SUM_NONE && a.ntx >= 50 &&
+        a.np > 128 * 64 && pass_table_bytes(a) >= BIG_TABLE && das_use_lds())
+        return false;
     // the cubic over 4 or more frames is staged in LDS (k_das_cubic_dma)
     return gk != GK_CUBIC || a.nfr < 4;
 }
@@ -127,16 +174,17 @@ int launch_das_wave(int gk, const DasArgs &a0, int max_part, float *partial, int
     // partial images (as many as the caller's workspace holds).
     const int64_t waves = ntiles * nw * passes;
     const int shares = w.split_inner ? no : (no + nw - 1) / nw;
-    int64_t nchunk = std::min<int64_t>((4096 + waves - 1) / waves, shares);
-    if (sum == WS_BOTH) nchunk = std::min<int64_t>(nchunk, partial ? max_part : 1);
-    // Four or more frames read a table too large for the L2s (every XCD would
-    // pull most of it): each XCD takes an eighth of the outer elements instead.
-    // 11 x 127 x 201 x 333, k-order, 12 frames: 600 -> 445 us.
-    if (a.nfr >= 4 && !w.split_inner && sum != WS_NONE && a.np <= (int64_t)1 << 24 &&
-        (sum != WS_BOTH || (partial && max_part >= 8))) {
-        w.slab = 1;
-        nchunk = 8;
+    int64_t target = 4096;
+    if (a.nfr >= 4 && !w.split_inner && a.np <= (int64_t)1 << 24) {
+        w.slab = wave_slab(gk, a, sum, no, ni, ntiles, passes) &&
+                 (sum != WS_BOTH || (partial && max_part >= 8));
+        // sums over frames wait on longer loads: 31 x 64 x 1000 onto 4800 pixels, 16
+        // frames, nearest per receiver: 4096 / 8192 / 16384 waves 155 / 123 / 107 us
+        if (sum != WS_NONE) target = 16384;
     }
+    int64_t nchunk = std::min<int64_t>((target + waves - 1) / waves, shares);
+    if (sum == WS_BOTH) nchunk = std::min<int64_t>(nchunk, partial ? max_part : 1);
+    if (w.slab) nchunk = 8;
     float *final_out = a.out;
     if (sum == WS_BOTH && nchunk > 1) a.out = partial;
     const size_t lds = std::max(wave_lds_bytes(w.ib, w.weights, nw), (size_t)nw * fc * 64 * 4);

@@ -158,6 +158,35 @@ def test_wave_gather_geometry_equals_its_tables(kind, nfr, thresh):
     assert (thresh > 1.0) == (not np.any(b))
 
 
+# which order and kernel a call over several frames takes: chunks of the outer axis
+# per XCD (few tiles; per-sample outputs of a geometry; one transmit, 13 frames and
+# more), finer chunks of it (few or many outer elements, small tables), and the
+# staged gather (nearest, 9 frames of a table over 96 MB)
+@pytest.mark.parametrize("ntx,nrx,nx,nz,nt,nfr,kind,sumtype,geo", [
+    (9, 20, 12, 25, 300, 5, "linear", "none", True), (9, 20, 12, 25, 300, 5, "linear", "none", False),
+    (1, 24, 65, 65, 300, 13, "nearest", "tx_only", True), (1, 24, 65, 65, 300, 12, "nearest", "tx_only", True),
+    (3, 20, 10, 21, 300, 4, "linear", "rx_only", True), (17, 20, 10, 21, 300, 4, "korder_cubic", "rx_only", False),
+    (9, 40, 65, 65, 300, 6, "linear", "tx_and_rx", True), (9, 15, 30, 30, 300, 4, "korder_cubic", "tx_and_rx", False),
+    (9, 40, 20, 30, 300, 8, "nearest", "tx_and_rx", False), (50, 64, 97, 85, 2000, 9, "nearest", "tx_and_rx", True)])
+def test_frame_batches_in_every_order(ntx, nrx, nx, nz, nt, nfr, kind, sumtype, geo, monkeypatch):
+    """Every order of a frame batch against the kernel that adds each sample by
+    itself; 1e-5 of the image peak (summation order)."""
+    _, _, pnts = sim.grid(nx, nz, (-4e-3, 4e-3), (2e-3, 0.9 * nt * DT * sim.C0 / 2))
+    steers = np.radians(np.linspace(-8, 8, ntx)) if ntx > 1 else np.zeros(1)
+    kw = dict(t0=0.0, dt=DT, nt=nt, interp={"kind": kind}, sumtype=sumtype)
+    if kind == "korder_cubic":
+        kw["interp"]["k"] = 8
+    bf = SyntheticBeamformer(**sim.pw_synthetic(steers, sim.linear_array(nrx), pnts), **kw)
+    if not geo:
+        t = bf.tables()
+        bf = TabbedBeamformer(tautx=t[0], apodtx=t[1], taurx=t[2], apodrx=t[3], **kw)
+    rf = np.random.default_rng(ntx + nt).standard_normal((nfr, ntx, nrx, nt)).astype(np.float32)
+    print(f"batch {ntx}x{nrx}x{nt} {nx * nz} px nfr={nfr} {kind} {sumtype} geo={geo}", flush=True)
+    got = bf(rf)
+    monkeypatch.setenv("PYCBF_DAS_PLAIN", "1")
+    assert_close_to_peak(got, bf(rf), 1e-5, sumtype)
+
+
 @pytest.mark.parametrize("nx,nz,xfast", [(13, 320, False), (64, 64, False), (37, 200, True), (4099, 1, False)])
 def test_wave_gather_over_grids_in_their_own_order(nx, nz, xfast):
     """Tables handed over in the pixels' own order (das_tabbed): grids of z or
