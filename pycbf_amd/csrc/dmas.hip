@@ -12,6 +12,9 @@
 // those two instructions per pair and by the column reads.  96 elements x
 // 60 000 pixels x 10 lags: 251 -> 20 us (k_dmas before: two reads through
 // L1, a product and a square root per pair).
+//
+// k_dmas, a lane per pixel, takes the columns that do not fit LDS and short ones
+// of many pixels (dmas_short).
 #include <math.h>
 
 #include "common.h"
@@ -161,13 +164,27 @@ __global__ __launch_bounds__(64 * DW) void k_dmas_cols(const float *__restrict__
     }
 }
 
+// Columns so short that holding them costs more than it saves: k_dmas_cols
+// launches four waves per 64 pixels, which many pixels pay for (times over those
+// of k_dmas, signed roots, lags 1 .. nsep - 1, summed / apart; n pixels in all):
+//   nsep 2: 1.2 at 1000, 3.1 at 1.6 M;  nsep 3: 1.08 / 0.97 at 4000, 1.3 at 100 000
+//   nsep 5: 0.9 / 0.7 at 20 000, 1.5 / 1.25 at 400 000, 1.9 / 1.6 at 1.6 M
+//   nsep 7: 0.9 / 0.8 at 100 000, 1.2 / 1.0 at 400 000, 1.4 / 1.1 at 1.6 M
+//   nsep 9: 0.8 / 0.6 at 100 000, 1.04 / 0.8 at 400 000;  nsep 12: 0.8 / 0.6 at 1.6 M
+static bool dmas_short(int64_t nsep, int64_t n, int sumlags)
+{
+    return nsep < 3 || (nsep <= (sumlags ? 9 : 6) && n >= 32768 * (nsep - 2));
+}
+
 int launch_dmas(const float *im, int64_t nfr, int64_t nsep, int64_t np, const int32_t *lags,
                 int nlag, int dmastype, int sumlags, float *out, hipStream_t s)
 {
     const int64_t n = nfr * np;
     if (n <= 0) return 0;
-    // columns too tall for LDS, or more frames than a grid axis: through L1
-    if (nsep <= DMAX_SEP - DW && nfr <= 65535 && np <= (int64_t)1 << 30) {
+    // columns too tall for LDS or too short for it, or more frames than a grid axis:
+    // through L1
+    if (nsep <= DMAX_SEP - DW && nfr <= 65535 && np <= (int64_t)1 << 30 &&
+        !dmas_short(nsep, n, sumlags)) {
         const dim3 grid((unsigned)((np + 63) / 64), (unsigned)nfr);
         hipLaunchKernelGGL(k_dmas_cols, grid, dim3(64 * DW), (size_t)(nsep + DW) * 256, s, im,
                            (int)nsep, np, lags, nlag, dmastype, sumlags, out);

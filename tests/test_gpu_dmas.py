@@ -92,6 +92,22 @@ def test_dmas_columns_and_lags_at_their_edges(nsep, npx, nfr):
                                      f"{nsep} {dmastype} {sumlags}")
 
 
+@pytest.mark.parametrize("nsep,npx,nfr", [(2, 40, 1), (3, 16384, 2), (3, 32767, 1), (6, 65537, 2), (6, 131071, 1),
+                                          (9, 57344, 4), (10, 70000, 4)])
+def test_dmas_of_short_columns(nsep, npx, nfr):
+    """Columns of few elements on both sides of the pixel count from which each
+    lane walks its own; lags apart leave the columns at another height.  Bar as
+    above."""
+    im = np.random.default_rng(nsep).standard_normal((nfr, nsep, npx)).astype(np.float32)
+    lags = list(range(1, nsep))
+    for dmastype in ("ssr", "power", "pssr"):
+        for sumlags in (True, False):
+            got = _dmas(im, lags, dmastype, sumlags)
+            for f in range(nfr):
+                assert_close_to_peak(got[f], numerics.dmas(im[f], lags, dmastype, sumlags), 1e-5,
+                                     f"{nsep} {dmastype} {sumlags}")
+
+
 def test_dmas_of_infinities_and_nans():
     """Infinite, NaN and zero elements count as in the column-free kernel, which
     the same columns padded with zeros to 300 elements take."""
