@@ -271,17 +271,15 @@ static int run_das(const pycbf_rfinfo *info, const float *rf, int64_t nfr, const
     // delay residuals: the direct gather places samples in double
     if (ttx_lo || trx_lo) return launch_das(plan.gk, a, plan.nsplit, part, s);
     if (das_use_plain()) return launch_das_plain(plan.gk, a, s);
+    // PYCBF_DAS_LDS=0: every call over delay tables, read straight from memory
+    if (!plan.bounds) return launch_das(plan.gk, a, plan.nsplit, part, s);
+    float *bnd = (float *)cv.take(plan.bounds);
     if (das_wave_applies(plan.gk, a))
-        return launch_das_wave(plan.gk, a, part ? plan.nsplit : 1, part,
-                               plan.bounds ? (int *)cv.take(plan.bounds) : nullptr, s);
-    if (plan.bounds) {
-        float *bnd = (float *)cv.take(plan.bounds);
-        if (!bnd) return fail(PYCBF_EINVAL, "workspace too small");
-        if ((rc = launch_tile_bounds(a, bnd, s))) return rc;
-        a.bounds = bnd;
-        return launch_das_lds(plan.gk, a, plan.nsplit, part, s);
-    }
-    return launch_das(plan.gk, a, plan.nsplit, part, s);
+        return launch_das_wave(plan.gk, a, part ? plan.nsplit : 1, part, (int *)bnd, s);
+    if (!bnd) return fail(PYCBF_EINVAL, "workspace too small");
+    if ((rc = launch_tile_bounds(a, bnd, s))) return rc;
+    a.bounds = bnd;
+    return launch_das_lds(plan.gk, a, plan.nsplit, part, s);
 }
 
 // Tries every significand of [1, 2); rounding to nearest is symmetric in the sign.

@@ -66,7 +66,7 @@ bool das_wave_applies(int gk, const DasArgs &a)
     // 128 tiles and fewer, or few transmits, this one is faster all the same (31 x
     // 128 x 2048 onto 64 x 64: 0.56 of it).
     if (gk == GK_NEAREST && a.nfr > 8 && a.sumflag != PYCBF_SUM_NONE && a.ntx >= 50 &&
-        a.np > 128 * 64 && pass_table_bytes(a) >= BIG_TABLE && das_use_lds())
+        a.np > 128 * 64 && pass_table_bytes(a) >= BIG_TABLE)
         return false;
     // the cubic over 4 or more frames is staged in LDS (k_das_cubic_dma)
     return gk != GK_CUBIC || a.nfr < 4;

@@ -187,6 +187,41 @@ def test_frame_batches_in_every_order(ntx, nrx, nx, nz, nt, nfr, kind, sumtype, 
     assert_close_to_peak(got, bf(rf), 1e-5, sumtype)
 
 
+@pytest.mark.parametrize("nfr", [None, 3, 9])
+def test_direct_gather_by_its_own_order(nfr, monkeypatch):
+    """PYCBF_DAS_LDS=0 selects the direct gather for every call: with unit weights
+    its sums are the per-sample values added one after the other, receivers (per
+    transmit) first, the transmits' sums then in order, bit for bit."""
+    rng = np.random.default_rng(11)
+    ntx, nrx, npx, nt = 5, 9, 300, 200
+    tabs = [(rng.uniform(0, 0.4, (n, npx)) * nt * DT).astype(np.float32) for n in (ntx, nrx)]
+    tabs = (tabs[0], np.ones((ntx, npx), np.float32), tabs[1], np.ones((nrx, npx), np.float32))
+    rf = rng.standard_normal((nfr or 1, ntx, nrx, nt)).astype(np.float32)
+    s = np.stack([oracle.das_tabbed(r, 0.0, DT, *tabs, kind="linear", sumtype="none") for r in rf])
+    add = lambda x, axis: np.add.accumulate(x, axis=axis, dtype=np.float32).take(-1, axis=axis)  # noqa: E731
+    per_tx = add(s, 2)
+    ref = {"tx_and_rx": add(per_tx, 1), "tx_only": add(s, 1), "rx_only": per_tx, "none": s}
+    monkeypatch.setenv("PYCBF_DAS_LDS", "0")
+    for sumtype, want in ref.items():
+        print(f"direct gather nfr={nfr} {sumtype}", flush=True)
+        got = _beamformer(tabs, 0.0, nt, {"kind": "linear"}, sumtype)(rf if nfr else rf[0])
+        assert np.array_equal(got, want if nfr else want[0]), sumtype
+
+
+def test_direct_gather_of_a_geometry(monkeypatch):
+    """The same switch over a point geometry: its delay tables, bit for bit."""
+    p = sim.pw_synthetic(np.radians(np.linspace(-10, 10, 4)), sim.linear_array(12),
+                         sim.grid(9, 37, (-4e-3, 4e-3), (2e-3, 9e-3))[2])
+    rf = np.random.default_rng(4).standard_normal((2, 4, 12, 600)).astype(np.float32)
+    monkeypatch.setenv("PYCBF_DAS_LDS", "0")
+    for kind in ("nearest", "cubic", "korder_cubic"):
+        kw = dict(t0=0.0, dt=DT, nt=600, interp={"kind": kind})
+        syn = SyntheticBeamformer(**p, **kw)
+        t = syn.tables()
+        tab = TabbedBeamformer(tautx=t[0], apodtx=t[1], taurx=t[2], apodrx=t[3], **kw)
+        assert np.array_equal(syn(rf), tab(rf)) and syn(rf).any(), kind
+
+
 @pytest.mark.parametrize("nx,nz,xfast", [(13, 320, False), (64, 64, False), (37, 200, True), (4099, 1, False)])
 def test_wave_gather_over_grids_in_their_own_order(nx, nz, xfast):
     """Tables handed over in the pixels' own order (das_tabbed): grids of z or
