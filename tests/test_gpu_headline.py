@@ -297,3 +297,37 @@ def test_dma_gather_wide_and_narrow_windows():
     for f in (0, 4, 9):
         ref, _ = oracle.das_tabbed_mt(rf[f], 0.0, dt, *tabs, kind="cubic")
         assert_close_to_peak(got[f], ref, 1e-5, f"wide/narrow frame {f}")
+
+
+@pytest.mark.parametrize("env", [{"PYCBF_DAS_DMA": "0"}, {"PYCBF_XCD_REMAP": "0"},
+                                 {"PYCBF_DAS_DMA": "0", "PYCBF_XCD_REMAP": "0"}], ids=lambda e: "+".join(sorted(e)))
+@pytest.mark.parametrize("nfr", [5, 10])
+def test_staged_gathers_wide_and_narrow_windows(nfr, env, monkeypatch):
+    """The staged gathers of a cubic batch of 4 frames and more, with the windows
+    staged through registers (PYCBF_DAS_DMA=0) and in round-robin workgroup order
+    (PYCBF_XCD_REMAP=0): channel windows within the 16-frame slots (95 and 160
+    entries) and past both, whose channels take the direct gather.  Summed images
+    and per-sample outputs against the oracle."""
+    ntx, nrx, nt = 5, 31, 1024
+    dt = 1.0 / sim.FS
+    steers = np.radians(np.linspace(-12, 12, ntx))
+    fx, fz = np.meshgrid(np.linspace(-0.3e-3, 0.3e-3, 32), np.linspace(20e-3, 20.45e-3, 16))
+    cx, cz = np.meshgrid(np.linspace(-5e-3, 5e-3, 32), np.linspace(4e-3, 12e-3, 16))
+    pnts = np.ascontiguousarray(np.stack([np.concatenate([fx.ravel(), cx.ravel()]),
+                                          np.concatenate([fz.ravel(), cz.ravel()])], axis=1))
+    p = sim.pw_synthetic(steers, sim.linear_array(nrx), pnts)
+    tabs = oracle.synthetic_tables(p["ovectx"], p["nvectx"], p["t0tx"], p["alatx"], p["doftx"],
+                                   p["ovecrx"], p["nvecrx"], p["alarx"], p["c0"], pnts)
+    rf = np.random.default_rng(18).standard_normal((nfr, ntx, nrx, nt)).astype(np.float32)
+    for k, v in env.items():
+        monkeypatch.setenv(k, v)
+    for sumtype in ("tx_and_rx", "tx_only", "none"):
+        print(f"staged gather {env} nfr={nfr} {sumtype}", flush=True)
+        bf = SyntheticBeamformer(**p, t0=0.0, dt=dt, nt=nt, interp={"kind": "cubic"}, sumtype=sumtype,
+                                 device="cuda:0")
+        win = _windows(tabs, bf._perm.cpu().numpy(), dt, 1)
+        assert np.nanmax(win) > 160 and np.nanmin(win) <= 95
+        got = bf(rf)
+        for f in (0, 4, nfr - 1):
+            ref = oracle.das_tabbed(rf[f], 0.0, dt, *tabs, kind="cubic", sumtype=sumtype)
+            assert_close_to_peak(got[f], ref, 1e-5, f"{sumtype} frame {f}")
