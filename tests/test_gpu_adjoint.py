@@ -351,3 +351,19 @@ def test_rf_adjoint_where_float32_does_not_resolve_the_samples(kind):
     lhs = 1.99 * float(out.detach().double().sum())
     terms = rf.detach().double() * grf.double()
     assert abs(lhs - float(terms.sum())) <= 1e-5 * float(terms.abs().sum()), (lhs, float(terms.sum()))
+
+
+@pytest.mark.parametrize("kind", ["nearest", "linear", "cubic", "korder_cubic"])
+def test_adjoint_with_divisions(kind):
+    """Half a nanosecond per sample, below the steps whose reciprocal is tried:
+    quotients by division in every adjoint kernel.  Bar: 1e-4 of the FP64
+    gradient's peak, as above."""
+    arrs = list(_case(43, ntx=9, nrx=8, np_=300, nfr=2))
+    arrs, t0, dt = arrs[:5], 2e-8, 5e-10
+    arrs[1], arrs[3] = arrs[1] * np.float32(0.02), arrs[3] * np.float32(0.02)
+    gout = np.random.default_rng(44).standard_normal((2, 300)).astype(np.float32)
+    out, g = _grads_gpu(arrs, t0, dt, kind, "tx_and_rx", 1e-2, gout)
+    ref_out, gr = _grads_ref(arrs, t0, dt, kind, "tx_and_rx", 1e-2, gout)
+    assert np.max(np.abs(out - ref_out)) <= 1e-4 * np.max(np.abs(ref_out))
+    for name, a, b in zip(NAMES, g, gr):
+        assert np.max(np.abs(a - b)) <= 1e-4 * np.max(np.abs(b)), name

@@ -175,3 +175,31 @@ def test_batch_without_a_finite_trace_start(t0):
     batch.run()
     torch.cuda.synchronize()
     assert not any(bool(o.any()) for o in batch.outputs)
+
+
+def test_batch_with_divisions():
+    """Half a nanosecond per sample, below the steps whose reciprocal is tried:
+    quotients by division, few and many transmits, against the oracle's Tabbed DAS
+    on the geometry's own tables (1e-5 of the peak)."""
+    import torch
+    import oracle
+    from pycbf_amd import sim
+    from pycbf_amd.gpu import SyntheticBeamformer
+    from pycbf_amd.gpu.batch import BatchRequest, RaggedBatch
+    dt, nt, f = 5e-10, 500, 5e-10 * sim.FS  # positions scale with the step
+    reqs, tabs = [], []
+    for ntx, nrx, nx, nz in ((2, 20, 5, 7), (9, 8, 12, 9)):
+        _, _, pnts = sim.grid(nx, nz, (-2e-3 * f, 2e-3 * f), (2e-3 * f, 7e-3 * f))
+        p = sim.pw_synthetic(np.radians(np.linspace(-9, 9, ntx)), sim.linear_array(nrx) * f, pnts)
+        reqs.append(BatchRequest(params=p, gridshape=(nx, nz)))
+        bf = SyntheticBeamformer(**p, t0=0.0, dt=dt, nt=nt, interp={"kind": "cubic"})
+        tabs.append([t.cpu().numpy() for t in bf.tables()])
+    batch = RaggedBatch(reqs, nt=nt, dt=dt)
+    batch.rf_all.normal_()
+    print("ragged batch with divisions", flush=True)
+    batch.run()
+    torch.cuda.synchronize()
+    for t, v, o in zip(tabs, batch.rf_views, batch.outputs):
+        ref = oracle.das_tabbed(v.cpu().numpy(), 0.0, dt, *t, kind="cubic").reshape(o.shape)
+        assert np.abs(ref).max() > 0
+        assert np.abs(o.cpu().numpy() - ref).max() <= 1e-5 * np.abs(ref).max()

@@ -187,6 +187,69 @@ def test_frame_batches_in_every_order(ntx, nrx, nx, nz, nt, nfr, kind, sumtype, 
     assert_close_to_peak(got, bf(rf), 1e-5, sumtype)
 
 
+@pytest.mark.parametrize("interp,usf", KINDS, ids=[k[0]["kind"] + str(k[1]) for k in KINDS])
+@pytest.mark.parametrize("ntx,nrx,npx,nfr,t0", [(3, 12, 70, None, 0.0), (9, 10, 130, 5, 3e-8), (9, 10, 130, 2, 0.0)])
+def test_wave_gather_with_divisions(ntx, nrx, npx, nfr, t0, interp, usf, monkeypatch):
+    """Half a nanosecond per sample, below the steps whose reciprocal is tried
+    (2^-30): quotients by division, integer row offsets.  Bars as above."""
+    dt, nt = 5e-10, 120
+    rng = np.random.default_rng(ntx + npx)
+    tabs = list(_tables(ntx, nrx, npx, nt, 0.0, False, rng))
+    tabs[0] = (tabs[0] * np.float32(dt / DT) + np.float32(t0)).astype(np.float32)
+    tabs[2] = (tabs[2] * np.float32(dt / DT)).astype(np.float32)
+    rf = rng.standard_normal((nfr or 1, ntx, nrx, nt)).astype(np.float32)
+    monkeypatch.setitem(globals(), "DT", dt)  # of the oracle and the beamformers here
+    for sumtype in ("tx_and_rx", "tx_only", "rx_only", "none"):
+        print(f"divisions {interp} {ntx}x{nrx} nfr={nfr} {sumtype}", flush=True)
+        got = _beamformer(tabs, t0, nt, interp, sumtype)(rf if nfr else rf[0])
+        ref = _reference(rf, t0, tabs, interp, usf, sumtype, monkeypatch).reshape(got.shape)
+        if sumtype == "none" and interp["kind"] in ("nearest", "linear") and usf == 1:
+            assert np.array_equal(got, ref)
+        else:
+            assert_close_to_peak(got, ref, 1e-5, sumtype)
+
+
+@pytest.mark.parametrize("kind", ["linear", "cubic", "korder_cubic", "akima"])
+@pytest.mark.parametrize("nt", [60, 69])
+def test_last_sample_time_past_the_last_knot(nt, kind, monkeypatch):
+    """The late starts of the nearest test: at 69 samples the last time lies a
+    whole sample past the last knot, whose index is clamped.  Against the kernel
+    that places each sample by itself."""
+    t0 = 0.5
+    rng = np.random.default_rng(nt)
+    last = np.float32(t0) + np.float32(DT) * np.float32(nt - 1)
+    tautx = np.linspace(t0, last, 70, dtype=np.float32)[None].repeat(9, axis=0)
+    tautx[:, ::4] = last
+    tabs = (tautx, np.ones_like(tautx), np.zeros((4, 70), np.float32), np.ones((4, 70), np.float32))
+    rf = rng.standard_normal((9, 4, nt)).astype(np.float32)
+    interp = {"kind": kind, "k": 8} if kind == "korder_cubic" else {"kind": kind}
+    for sumtype in ("tx_and_rx", "tx_only", "none"):
+        got = _beamformer(tabs, t0, nt, interp, sumtype)(rf)
+        monkeypatch.setenv("PYCBF_DAS_PLAIN", "1")
+        ref = _beamformer(tabs, t0, nt, interp, sumtype)(rf)
+        monkeypatch.delenv("PYCBF_DAS_PLAIN")
+        assert_close_to_peak(got, ref, 1e-5, sumtype)
+
+
+@pytest.mark.parametrize("interp,usf", [k for k in KINDS if k[0]["kind"] != "makima" and k[1] == 1],
+                         ids=lambda v: v["kind"] if isinstance(v, dict) else "")
+@pytest.mark.parametrize("nt", [2 ** 19, 2 ** 19 + 1])
+def test_longest_float_offsets(nt, interp, usf, monkeypatch):
+    """Traces at and one past the entries whose byte offsets a float's low bits
+    hold, with delays among the last samples and at the last."""
+    rng = np.random.default_rng(nt)
+    last = np.float32(DT) * np.float32(nt - 1)
+    tautx = rng.uniform(0, last, (1, 130)).astype(np.float32)
+    tautx[0, 1::3] = last - (rng.uniform(0, 50, 43) * DT).astype(np.float32)
+    tautx[0, ::3] = last
+    tabs = (tautx, np.ones_like(tautx), np.zeros((2, 130), np.float32), np.ones((2, 130), np.float32))
+    rf = rng.standard_normal((1, 1, 2, nt)).astype(np.float32)
+    print(f"{nt} samples {interp}", flush=True)
+    for sumtype in ("tx_and_rx", "none"):
+        got = _beamformer(tabs, 0.0, nt, interp, sumtype)(rf[0])
+        assert_close_to_peak(got, _reference(rf, 0.0, tabs, interp, usf, sumtype, monkeypatch)[0], 1e-5, sumtype)
+
+
 @pytest.mark.parametrize("nfr", [None, 3, 9])
 def test_direct_gather_by_its_own_order(nfr, monkeypatch):
     """PYCBF_DAS_LDS=0 selects the direct gather for every call: with unit weights
