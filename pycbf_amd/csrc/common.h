@@ -105,7 +105,8 @@ int launch_das(int gk, const DasArgs &a, int nsplit, float *partial, hipStream_t
 // LDS-staged gather (delay tables or in-register synthetic geometry); bounds
 // must hold the tile delay ranges written by launch_tile_bounds.
 int launch_das_lds(int gk, const DasArgs &a, int nsplit, float *partial, hipStream_t s);
-// Wave-tile gather (das_wave.h): one wave per 64 pixels, samples through L1.
+// Wave-tile gather (das_wave.h): one wave per 64 pixels, samples through L1;
+// das_wave_applies says which calls it takes.
 // It may write up to max_part partial images (nfr, np) into `partial`, and an
 // int of scratch into `fast` (both may be null).
 bool das_wave_applies(int gk, const DasArgs &a);
@@ -120,9 +121,10 @@ int launch_tile_bounds(const DasArgs &a, float *bounds, hipStream_t s);
 inline int64_t das_tiles(int64_t np) { return (np + 255) / 256; }
 // out[g] = sum over z < nsplit of part[z*n + g]
 int launch_reduce_split(const float *part, int nsplit, int64_t n, float *out, hipStream_t s);
-// Whether the LDS-staged gather is used (PYCBF_DAS_LDS=0 selects the direct one).
+// False with PYCBF_DAS_LDS=0: every call without delay residuals takes the
+// direct gather too.
 bool das_use_lds();
-// Frames handled per pass of the gather (1, 2, 4, 8 or 16; PYCBF_DAS_FC caps it).
+// Frames per pass of the direct gather (1, 2, 4, 8 or 16; PYCBF_DAS_FC caps it).
 int das_frames_per_pass(int64_t nfr);
 // Whether transmits are the outer (one element per workgroup) axis.
 bool das_outer_is_tx(int sumflag, int64_t ntx, int64_t nrx);
@@ -177,7 +179,7 @@ struct BwdArgs {
 // trace's bins in LDS); else per pixel tile, which reads a.bounds.
 int bwd_per_channel(int gk, const BwdArgs &a, bool &yes);
 // gc0 (geo > 0, may be null): d loss / d c0, one float, reduced in a fixed order
-// from a.gc0part ((ntx + nrx) * das_tiles(np) doubles)
+// from a.gc0part ((ntx + nrx + 64) * das_tiles(np) doubles)
 int launch_das_bwd(int gk, const BwdArgs &a, float *gtautx, float *gapodtx, float *gtaurx,
                    float *gapodrx, float *grf, float *gc0, hipStream_t s);
 // Delay / apodisation gradients (and c0 partials) of one axis on wave tiles

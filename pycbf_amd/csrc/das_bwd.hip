@@ -14,11 +14,15 @@
 //   d tautx[tx, p]  = sum_f sum_rx G w v'(x)     d apodtx[tx, p] = sum_f sum_rx G apodrx v(x)
 //   d taurx[rx, p]  = sum_f sum_tx G w v'(x)     d apodrx[rx, p] = sum_f sum_tx G apodtx v(x)
 //   d rf[f, tx, rx, k] = sum_p G w dv(x)/dy_k                       (transposed gather)
-// k_das_bwd_tau evaluates the first four with one lane per (element, pixel),
-// recomputing x and w from the tables.  The channel-data gradient is a
+// The first four are k_bwd_elem's (das_bwd_elem.hip); k_das_bwd_tau, one lane
+// per (element, pixel), serves what that one does not take (one-sample linear
+// traces, nearest traces over 2^22 entries, images over 2^28 pixels, and c0
+// alone over an axis too long for LDS).  Both recompute x and w.  The
+// channel-data gradient is a
 // scatter into 64-bit fixed-point LDS bins (scale from k_bwd_scale's bound):
 // k_das_bwd_rf_ch (traces up to 4096 samples) gives each workgroup one
-// channel and writes its rows once; k_das_bwd_rf (longer traces) gives each
+// channel and writes its rows once, for the synthetic geometry from the delay
+// table of k_unit_delays; k_das_bwd_rf (longer traces) gives each
 // workgroup a (pixel tile, transmit, frame), bins the tile's sample window
 // per receive channel (k_tile_bounds) and flushes it with one float atomic
 // per non-zero bin.  For the natural

@@ -22,6 +22,12 @@
 //
 // The natural cubic with sums over 4 or 16 frames per pass runs
 // k_das_cubic_dma, which stages the same windows with LDS DMA (below).
+// k_das_lds serves what that one and the wave-tile gather (das_wave.h) leave:
+// the cubic over 4 frames and more with per-sample outputs, with more than 256
+// inner elements, or with a dt or c0 whose reciprocal form is not exact; large
+// nearest sums over 9 frames and more; and what does not fit a wave tile's
+// indexes (one-sample linear traces, nearest traces over 2^22 entries, images
+// over 2^28 pixels).
 #include <math.h>
 #include <stdlib.h>
 
@@ -454,9 +460,8 @@ typedef const __attribute__((address_space(1))) void glb_void;
 // the unlisted evaluations themselves: 16 frames of 75 x 128 x 4096 onto 512 x
 // 512 5.56 ms; without the weights and the acceptance test, 2.70e9 -> 2.28e9
 // VALU instructions, 5.48 ms; with the list, 1.91e9 VALU and 0.72e9 scalar
-// ones (1.54e9), 4.43 ms.)  What bounds it now: VALU issue, 80 % of the cycles,
-// and the LDS reads of the stencil.
-
+// ones (1.54e9), 4.43 ms.)  What bounds it now: VALU issue, 63 % of the cycles,
+// and bank conflicts of the stencil's LDS reads, 29 %.
 template <int SUM, int FC, int GEO, bool OUTER_TX, bool FODD, bool UNIT>
 __global__ __launch_bounds__(LDS_BLOCK) void k_das_cubic_dma(DasArgs A)
 {
@@ -862,7 +867,7 @@ static bool das_cubic_dma_enabled()
 }
 
 // frames per workgroup for the staged gather: 16 or 4 (fewer frames than 4
-// come here only when the wave-tile gather does not take the trace)
+// come here only when the wave-tile gather does not take the call)
 int das_lds_frames_per_pass(int64_t nfr)
 {
     int cap = 16;
