@@ -150,9 +150,11 @@ int launch_das_wave(int gk, const DasArgs &a0, int max_part, float *partial, int
     const int64_t passes = (a.nfr + fc - 1) / fc;
     // Waves per tile: the waves of a tile end together, so many small shares
     // leave more of them idle at its end, but few tiles need them to fill the
-    // chip.  1024 tiles (31 x 128 x 256 x 256, k-order): 171 us with 8 waves, 152
-    // with 16; 4096 tiles (75 x 128 x 512 x 512, cubic): 845 / 799 / 990 us with
-    // 4 / 8 / 16.
+    // chip.  8 and 16 waves, us (cubic): 31 x 128 x 2048, 512 tiles 102 / 82, 1024
+    // 128 / 118, 4096 360 / 346; 11 x 64 x 1024, 512 tiles 36 / 33, 1024 46 / 47,
+    // 4096 105 / 118; 75 x 128 x 512 x 512 799 / 990 (4 waves 845).  The line that
+    // suits an image moves up with the receivers that a wave walks and with its
+    // shape; this one, for all, is within 12 % of the better side.
     int nw = ntiles * passes > 1024 ? 8 : 16;
     w.group = 1;
     while (w.group < 32 && ntiles >= 64 * (int64_t)w.group) w.group *= 2;
