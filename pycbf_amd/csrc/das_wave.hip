@@ -154,7 +154,7 @@ int launch_das_wave(int gk, const DasArgs &a0, int max_part, float *partial, int
     // 128 / 118, 4096 360 / 346; 11 x 64 x 1024, 512 tiles 36 / 33, 1024 46 / 47,
     // 4096 105 / 118; 75 x 128 x 512 x 512 799 / 990 (4 waves 845).  The line that
     // suits an image moves up with the receivers that a wave walks and with its
-    // shape; this one, for all, is within 12 % of the better side.
+    // shape; this one, for all, is within 16 % of the better side.
     int nw = ntiles * passes > 1024 ? 8 : 16;
     w.group = 1;
     while (w.group < 32 && ntiles >= 64 * (int64_t)w.group) w.group *= 2;
